@@ -247,8 +247,9 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     st->stride = blob_stride;
     st->max_kv = max_kv;
 
-    // attention tiles / split items (the generic kernel of plain-layout pools
-    // takes one workgroup per (row, q head) and needs none)
+    // attention tiles / split items (plain-layout pools: column tiles for
+    // head_dim a multiple of 4, below; the scalar kernel of the others takes
+    // one workgroup per (row, q head) and needs none)
     const int G = ctx->q_per_kv, qpt = ctx->plain_kv ? 0 : 16 / G;
     st->h_tiles.clear();
     st->h_items.clear();
@@ -260,6 +261,20 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     if (!ctx->plain_kv && ctx->desc.kv_dtype == ZR_DTYPE_BF16 && G <= 32 && 32 % G == 0) prows = 128 / G;
     if (const char* env = getenv("ZR_ATTN_PREFILL"))
         if (atoi(env) == 0) prows = 0;
+    if (ctx->plain_kv && ctx->head_dim % 4 == 0) {
+        st->plain = plain_attention_plan(ctx->head_dim, ctx->local_kv_heads, G, mb->q_len, S);
+        const long width = 16L * st->plain.ct;
+        for (int s = 0; s < S; ++s) {
+            const long cols = (long)mb->q_len[s] * G;
+            for (long c0 = 0; c0 < cols; c0 += width) {
+                const int nc = (int)std::min(width, cols - c0);
+                const int last_visible = mb->kv_before[s] + (int)((c0 + nc - 1) / G);
+                const int pages = (mb->first_offset[s] + last_visible + 1 + kPageRows - 1) / kPageRows;
+                st->h_pblocks.push_back(make_int4(s, (int)c0, nc, pages));
+                st->h_psplits.push_back(make_int4(0, pages, -1, 1));
+            }
+        }
+    }
     std::vector<int> tile_pages;
     std::vector<int4> pblk;  // prefill blocks {seq, r0, nrows, pages}
     long total_pages = 0, total_ktiles = 0;

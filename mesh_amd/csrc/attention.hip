@@ -1186,8 +1186,9 @@ static zr_status launch_attn_t(zr_context* ctx, StagedMeta* st, int layer, const
 }
 
 // ------------------------------------------------------- any head_dim
-// Pools in the plain layout (head_dim other than 64 / 128, or q heads per kv
-// head not dividing 16): one wave per (query row, q head).  The wave walks
+// Pools in the plain layout whose head_dim is not a multiple of 4 (the rows of
+// a page are then not 8- / 16-byte aligned; attention_plain.hip serves the
+// others): one wave per (query row, q head).  The wave walks
 // the visible keys 64 at a time (a key per lane: the lane's score over D from
 // its K row; rows of a page are contiguous), keeps an online softmax across
 // the wave and accumulates P.V with lanes over the dims (up to 4 per lane).
@@ -1447,6 +1448,7 @@ zr_status launch_attention(zr_context* ctx, StagedMeta* st, int layer, const flo
     if (st->total_q == 0) return ZR_OK;
     if (ctx->plain_kv) {
         if (ctx->head_dim > 256) return set_err(ctx, ZR_E_UNSUPPORTED, "head_dim %d above 256", ctx->head_dim);
+        if (ctx->head_dim % 4 == 0) return launch_attention_plain(ctx, st, layer, q, out, out_bf16);
         return ctx->desc.kv_dtype == ZR_DTYPE_BF16
                    ? launch_attn_generic<uint16_t>(ctx, st, layer, q, out, out_bf16)
                    : launch_attn_generic<float>(ctx, st, layer, q, out, out_bf16);

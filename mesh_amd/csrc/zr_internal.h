@@ -288,6 +288,13 @@ constexpr int kTimingClasses = 5;
 void timing_mark_begin(zr_context* ctx, int cls, hipEvent_t* out);
 void timing_mark_end(zr_context* ctx, int cls, hipEvent_t begin);
 
+// Tile width (ct x 16 columns) and waves per workgroup of the plain-layout
+// attention launch (attention_plain.hip), fixed when a microbatch is staged.
+struct PlainAttnPlan {
+    int ct = 1, waves = 4;
+};
+PlainAttnPlan plain_attention_plan(int head_dim, int kv_heads, int G, const int* q_len, int n);
+
 // Staged microbatch metadata (device) ------------------------------------
 struct StagedMeta {
     zr_context* ctx = nullptr;
@@ -297,7 +304,8 @@ struct StagedMeta {
     int n_attn_items = 0;     // attention work items (per kv head)
     int n_tiles = 0;          // attention query tiles (per kv head)
     int n_merge = 0;          // tiles with more than one split
-    int n_pblocks = 0;        // prefill work units (block, key split) per kv head
+    int n_pblocks = 0;        // prefill work units (block, key split) per kv head; plain layout: tiles
+    PlainAttnPlan plain;      // plain layout with head_dim a multiple of 4
     int prefill_kh = 1;       // key halves per prefill workgroup (1: 4 waves, 2: 8 waves)
     int n_part_items = 0;     // partial items: decode items, then prefill (group, split) items
     bool pure_decode = false; // every sequence has one query row (MFMA page layout): RoPE + KV append can run
@@ -329,7 +337,8 @@ struct StagedMeta {
     //   {the pool pages of the item's first 4 pages (the last one repeated past its end)}
     int4* attn_rec = nullptr;
     int4* merge_rec = nullptr;  // [n_merge] tiles the merge kernel combines: {first partial, splits, first q row, nq}
-    int4* pblocks = nullptr;    // [n_pblocks] {seq, r0, nrows, pages}, most key tiles first
+    int4* pblocks = nullptr;    // [n_pblocks] {seq, r0, nrows, pages}, most key tiles first (plain layout:
+                                // {seq, first column, columns, pages}, column = row x q heads per kv head + head)
     int4* psplits = nullptr;    // [n_pblocks] {first key tile, end key tile, item, splits}
     // host copies
     std::vector<int> h_q_len, h_kv_before, h_first_pos, h_first_offset, h_block_tables;
@@ -393,6 +402,9 @@ zr_status launch_rope_kv_write(zr_context* ctx, StagedMeta* st, int layer, const
 // out_f32 [T, q_cols] or out_bf16 (A operand of the O projection).
 zr_status launch_attention(zr_context* ctx, StagedMeta* st, int layer, const float* q, float* out_f32,
                            uint16_t* out_bf16);
+// Plain-layout pools with head_dim a multiple of 4 (tiles staged in pblocks).
+zr_status launch_attention_plain(zr_context* ctx, StagedMeta* st, int layer, const float* q, float* out_f32,
+                                 uint16_t* out_bf16);
 // Pure decode microbatches (st->pure_decode): RoPE + KV append and attention in
 // one launch, q and the new K / V rows read from the QKV product's slabs.
 // Times `repeats` launches of a read-only copy of the decode attention
