@@ -1465,6 +1465,41 @@ static zr_status kv_copy_entry(zr_context* ctx, const int* block_table, int n_pa
 
 }  // extern "C"
 
+namespace zr {
+
+zr_status kv_stage_rows(zr_context* ctx, int n_rows, float** d_k, float** d_v) {
+    ZR_HIP(ctx, hipSetDevice(ctx->device));
+    const size_t elems = (size_t)ctx->desc.num_layers * n_rows * ctx->kv_cols;
+    const size_t need = 2 * elems + (size_t)n_rows / kPageRows + 2;  // a partial first page: one page more
+    if (need > ctx->kv_stage_floats) {
+        ZR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (ctx->kv_stage) (void)hipFree(ctx->kv_stage);
+        ctx->kv_stage = nullptr;
+        ctx->kv_stage_floats = 0;
+        ZR_HIP(ctx, hipMalloc(&ctx->kv_stage, need * sizeof(float)));
+        ctx->kv_stage_floats = need;
+    }
+    *d_k = ctx->kv_stage;
+    *d_v = ctx->kv_stage + elems;
+    return ZR_OK;
+}
+
+zr_status kv_scatter_staged(zr_context* ctx, const int* block_table, int n_pages, int first_offset, int n_rows) {
+    if (zr_status rc = kv_copy_check(ctx, block_table, n_pages, first_offset, 0, n_rows)) return rc;
+    const int L = ctx->desc.num_layers;
+    const size_t elems = (size_t)L * n_rows * ctx->kv_cols;
+    // the pages the rows touch: the room kv_stage_rows keeps for the table
+    const int used = (first_offset + n_rows - 1) / kPageRows + 1;
+    int* d_table = (int*)(ctx->kv_stage + 2 * elems);
+    ZR_HIP(ctx, hipMemcpyAsync(d_table, block_table, 4 * (size_t)used, hipMemcpyHostToDevice, ctx->stream));
+    if (zr_status rc = launch_kv_copy(ctx, 0, L, d_table, first_offset, 0, n_rows, ctx->kv_stage, ctx->kv_stage + elems, 1))
+        return rc;
+    ZR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return ZR_OK;
+}
+
+}  // namespace zr
+
 // One session window's KV in a device buffer of its own, on its way to or
 // from host memory on a copy stream: K [layers][rows][kv_cols], then V, then
 // room for a page table.  `used` is recorded after the last compute-stream

@@ -3,9 +3,10 @@
 // export: the bytes KVCache::to_bytes (kv_cache.rs:880-887; ciborium 0.2.2,
 // Cargo.lock:627-629) writes for the cache DeviceKVCache::export_snapshot
 // (forward_pass.rs:1169-1204) builds, encoded from the gathered K / V rows.
-// import: a host decoder of the same document (import_snapshot,
-// forward_pass.rs:1206-1242, reads it back through KVCache::from_bytes,
-// kv_cache.rs:889-895).
+// import: a decoder of the same document on the device, and a strict reader on
+// the host for every other form serde accepts and for the errors
+// (import_snapshot, forward_pass.rs:1206-1242, reads it back through
+// KVCache::from_bytes, kv_cache.rs:889-895).
 //
 // Document (serde derive: a struct is a definite map of field-name text ->
 // value in declaration order; None = null; usize = unsigned integer; Vec =
@@ -496,6 +497,370 @@ zr_status launch_kv_cbor(zr_context* ctx, const float* d_k, const float* d_v, in
     timing_mark_end(ctx, kClassKvCbor, ev);
     ZR_HIP(ctx, hipMemcpyAsync(out, ctx->cbor_out, doc, hipMemcpyDeviceToHost, ctx->stream));
     ZR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return ZR_OK;
+}
+
+// ------------------------------------------------- decoder on the device --
+// Reads the document kv_cbor_layout describes (what KVCache::to_bytes and the
+// encoder above write) without walking it on the host.  Its items are flat --
+// no byte string, and every head is followed by its items -- so an item's
+// length follows from its first byte alone, at most 14 (a 13-letter key).
+// Where items start is then a small automaton: a 64-byte segment maps the
+// offset (0..13) of its first item to the offset of the next segment's first
+// one, 14 nibbles in a word, and such maps compose:
+//   cbor_map_kernel     each thread's segment map by one backward pass (the map
+//                       of the last 16 positions slides along in the word), and
+//                       the block's maps composed by a scan;
+//   cbor_entry_kernel   the blocks' maps composed: each block's first item;
+//   cbor_tally_kernel   floats per thread and block, items that are no float
+//                       (then the encoder's two-level scan of the block counts);
+//   cbor_read_kernel    the floats, through LDS, into the K / V rows, and where
+//                       each of the 2L arrays starts and ends.
+// The host then compares the bytes outside the arrays with the layout's.  With
+// 2L n floats, the right bytes in every gap and no other item anywhere, each
+// array is n float items and the document is the one the strict reader below
+// accepts with these rows; anything else is left to that reader, errors and
+// all.  Bound by the copy of the bytes to the device, ~2 ms from pageable
+// memory for 69 MB (23M floats); the passes take 190 us: map 54, tally 27, read
+// 85, the three scans 22.
+namespace {
+
+constexpr int kTokSeg = 64;                       // bytes per thread
+constexpr int kTokThreads = 256;
+constexpr int kTokBlock = kTokSeg * kTokThreads;  // bytes per block
+constexpr int kTokFloats = kTokBlock / 3 + 1;     // floats that can start in a block
+
+// Bytes of the item that starts with b (1 for what the document never holds).
+__host__ __device__ inline int cbor_item_len(uint32_t b) {
+    const uint32_t major = b >> 5, info = b & 31;
+    if (info >= 24) return (int)((0x11119532u >> (4 * (info - 24))) & 15u);  // 1-, 2-, 4-, 8-byte argument
+    return (major == 2 || major == 3) && info <= 13 ? (int)info + 1 : 1;
+}
+
+struct TokArgs {
+    const uint8_t* doc;             // padded to whole blocks + 16
+    unsigned long long len;
+    int blocks;
+    unsigned long long* fn;         // [blocks][kTokThreads] maps of the block's bytes before the thread's
+    unsigned long long* block_fn;   // [blocks]
+    uint32_t* entry;                // [blocks] offset of the block's first item
+    uint8_t* thread_floats;         // [blocks][kTokThreads]
+    uint32_t* block_floats;         // [blocks]
+    unsigned long long* off;        // [blocks] floats before the block inside its group of 1024
+    unsigned long long* group_off;  // [groups + 1]
+    unsigned long long* others;     // items that are no float
+    unsigned long long* starts;     // [arrays] byte offset of the array's first float
+    unsigned long long* ends;       // [arrays] ... past its last float
+    int arrays;
+    unsigned long long n;           // floats per array
+    float* k;
+    float* v;
+};
+
+// The block's bytes and the 16 after them, a word of padding per segment (a
+// wave's 64 segments then start in different banks).
+struct TokBytes {
+    uint32_t w[kTokBlock / 4 + kTokThreads + 8];
+    __device__ inline void load(const TokArgs& a) {
+        const uint4* src = (const uint4*)(a.doc + (size_t)blockIdx.x * kTokBlock);
+        for (int q = threadIdx.x; q < kTokBlock / 16 + 1; q += kTokThreads) {
+            const uint4 x = src[q];
+            uint32_t* d = w + 4 * q + (q >> 2);
+            d[0] = x.x;
+            d[1] = x.y;
+            d[2] = x.z;
+            d[3] = x.w;
+        }
+        __syncthreads();
+    }
+    __device__ inline uint32_t at(uint32_t p) const { return (w[(p >> 2) + (p >> 6)] >> (8 * (p & 3))) & 0xffu; }
+};
+
+__device__ inline uint32_t map_at(unsigned long long f, uint32_t s) { return (uint32_t)(f >> (4 * s)) & 15u; }
+// the map "f, then g"
+__device__ inline unsigned long long map_then(unsigned long long f, unsigned long long g) {
+    unsigned long long r = 0;
+#pragma unroll
+    for (int s = 0; s < 14; ++s) r |= (unsigned long long)map_at(g, map_at(f, s)) << (4 * s);
+    return r;
+}
+constexpr unsigned long long kMapIdentity = 0xfedcba9876543210ull;
+
+// inclusive scan of the threads' maps; `buf` [2][threads]
+template <int THREADS>
+__device__ inline unsigned long long map_scan(unsigned long long f, unsigned long long (*buf)[THREADS]) {
+    const int t = threadIdx.x;
+    int cur = 0;
+    buf[0][t] = f;
+    __syncthreads();
+    for (int o = 1; o < THREADS; o <<= 1) {
+        if (t >= o) f = map_then(buf[cur][t - o], f);
+        buf[cur ^ 1][t] = f;
+        cur ^= 1;
+        __syncthreads();
+    }
+    return f;
+}
+
+__global__ __launch_bounds__(kTokThreads) void cbor_map_kernel(TokArgs a) {
+    __shared__ TokBytes b;
+    __shared__ unsigned long long buf[2][kTokThreads];
+    b.load(a);
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < a.arrays; i += kTokThreads) a.starts[i] = a.ends[i] = ~0ull;
+        if (threadIdx.x == 0) *a.others = 0;
+    }
+    unsigned long long f = kMapIdentity;  // nibble j: offset past the segment of an item at position p + 1 + j
+    const uint32_t* w = b.w + threadIdx.x * (kTokSeg / 4 + 1);
+#pragma unroll
+    for (int q = kTokSeg / 4 - 1; q >= 0; --q) {
+        const uint32_t x = w[q];
+#pragma unroll
+        for (int j = 3; j >= 0; --j) f = (f << 4) | map_at(f, cbor_item_len((x >> (8 * j)) & 0xffu) - 1);
+    }
+    f = map_scan(f, buf);
+    const size_t g = (size_t)blockIdx.x * kTokThreads + threadIdx.x;
+    if (threadIdx.x + 1 < kTokThreads) a.fn[g + 1] = f;
+    if (threadIdx.x == 0) a.fn[g] = kMapIdentity;
+    if (threadIdx.x + 1 == kTokThreads) a.block_fn[blockIdx.x] = f;
+}
+
+__global__ __launch_bounds__(1024) void cbor_entry_kernel(TokArgs a) {
+    __shared__ unsigned long long buf[2][1024];
+    const int per = (a.blocks + 1023) / 1024;
+    const int b0 = threadIdx.x * per, b1 = min(b0 + per, a.blocks);
+    unsigned long long f = kMapIdentity;
+    for (int i = b0; i < b1; ++i) f = map_then(f, a.block_fn[i]);
+    f = map_scan(f, buf);
+    buf[0][threadIdx.x] = f;
+    __syncthreads();
+    uint32_t s = threadIdx.x ? map_at(buf[0][threadIdx.x - 1], 0) : 0u;  // the document starts with an item
+    for (int i = b0; i < b1; ++i) {
+        a.entry[i] = s;
+        s = map_at(a.block_fn[i], s);
+    }
+}
+
+// Calls item(p, length, is_float) for every item that starts in the thread's
+// segment and inside the document (p: block offset); a float that the document
+// cuts short is none.
+template <typename F>
+__device__ inline void tok_walk(const TokArgs& a, const TokBytes& b, F item) {
+    const unsigned long long base = (unsigned long long)blockIdx.x * kTokBlock;
+    const uint32_t s0 = threadIdx.x * kTokSeg;
+    const size_t g = (size_t)blockIdx.x * kTokThreads + threadIdx.x;
+    uint32_t p = s0 + map_at(a.fn[g], a.entry[blockIdx.x]);
+    while (p < s0 + kTokSeg && base + p < a.len) {
+        const uint32_t x = b.at(p);
+        const uint32_t len = cbor_item_len(x);
+        item(p, len, x >= 0xf9u && x <= 0xfbu && base + p + len <= a.len);
+        p += len;
+    }
+}
+
+__global__ __launch_bounds__(kTokThreads) void cbor_tally_kernel(TokArgs a) {
+    __shared__ TokBytes b;
+    __shared__ uint32_t red[2][kTokThreads / 64];
+    b.load(a);
+    uint32_t floats = 0, others = 0;
+    tok_walk(a, b, [&](uint32_t, uint32_t, bool f) {
+        floats += f;
+        others += !f;
+    });
+    a.thread_floats[(size_t)blockIdx.x * kTokThreads + threadIdx.x] = (uint8_t)floats;  // at most 22
+    const uint32_t fsum = block_sum(floats, red[0]), osum = block_sum(others, red[1]);
+    if (threadIdx.x == 0) {
+        a.block_floats[blockIdx.x] = fsum;
+        if (osum) atomicAdd(a.others, (unsigned long long)osum);
+    }
+}
+
+// the f32 of a float item, as the strict reader below converts it
+__device__ inline float tok_value(const TokBytes& b, uint32_t p, uint32_t len) {
+    uint32_t hi = 0;
+    if (len == 3) {
+        const uint32_t h = (b.at(p + 1) << 8) | b.at(p + 2);
+        const uint32_t s = (h & 0x8000u) << 16, e = (h >> 10) & 0x1f, m = h & 0x3ff;
+        if (e == 0x1f) return __uint_as_float(s | 0x7f800000u | (m << 13));
+        if (e) return __uint_as_float(s | ((e + 112) << 23) | (m << 13));
+        // zero or a binary16 subnormal m * 2^-24: exact in f32
+        return __uint_as_float(s | __float_as_uint((float)m * 0x1p-24f));
+    }
+#pragma unroll
+    for (int i = 1; i <= 4; ++i) hi = (hi << 8) | b.at(p + i);
+    if (len == 5) return __uint_as_float(hi);
+    uint32_t lo = 0;
+#pragma unroll
+    for (int i = 5; i <= 8; ++i) lo = (lo << 8) | b.at(p + i);
+    if ((hi & 0x7ff00000u) == 0x7ff00000u && ((hi & 0xfffffu) | lo))  // NaN: quieted, the payload's top bits kept
+        return __uint_as_float((hi & 0x80000000u) | 0x7fc00000u | ((hi & 0xfffffu) << 3) | (lo >> 29));
+    return (float)__hiloint2double((int)hi, (int)lo);
+}
+
+__global__ __launch_bounds__(kTokThreads) void cbor_read_kernel(TokArgs a) {
+    __shared__ TokBytes b;
+    __shared__ float out[kTokFloats];
+    __shared__ uint32_t wsum[kTokThreads / 64];
+    b.load(a);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t mine = a.thread_floats[(size_t)blockIdx.x * kTokThreads + threadIdx.x];
+    uint32_t incl = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t before = incl - mine, total = 0;
+#pragma unroll
+    for (int w = 0; w < kTokThreads / 64; ++w) {
+        if (w < wave) before += wsum[w];
+        total += wsum[w];
+    }
+    const unsigned long long first = a.group_off[blockIdx.x >> 10] + a.off[blockIdx.x];  // floats before the block
+    const unsigned long long base = (unsigned long long)blockIdx.x * kTokBlock;
+    if (mine) {
+        const unsigned long long idx = first + before;
+        unsigned long long arr = idx / a.n, r = idx - arr * a.n;
+        uint32_t o = before;
+        tok_walk(a, b, [&](uint32_t p, uint32_t len, bool f) {
+            if (!f) return;
+            out[o++] = tok_value(b, p, len);
+            if (arr < (unsigned long long)a.arrays) {
+                if (r == 0) a.starts[arr] = base + p;
+                if (r + 1 == a.n) a.ends[arr] = base + p + len;
+            }
+            if (++r == a.n) {
+                r = 0;
+                ++arr;
+            }
+        });
+    }
+    __syncthreads();
+    const unsigned long long arr0 = first / a.n, r0 = first - arr0 * a.n;
+    for (uint32_t i = threadIdx.x; i < total; i += kTokThreads) {
+        unsigned long long arr = arr0, r = r0 + i;
+        while (r >= a.n) {  // n >= kTokMinArray: a block spans few arrays
+            r -= a.n;
+            ++arr;
+        }
+        if (arr < (unsigned long long)a.arrays) ((arr & 1) ? a.v : a.k)[(arr >> 1) * a.n + r] = out[i];
+    }
+}
+
+constexpr long long kTokMinArray = 512;
+
+// the four integers of the trailing config map, where it is the layout's
+bool tail_config(const uint8_t* bytes, size_t len, int cfg[4]) {
+    static const char* names[4] = {"num_layers", "num_heads", "head_dim", "max_seq_len"};
+    const uint8_t key[7] = {0x66, 'c', 'o', 'n', 'f', 'i', 'g'};
+    for (size_t back = 8; back <= 128 && back <= len; ++back) {
+        size_t i = len - back;
+        if (memcmp(bytes + i, key, 7) != 0) continue;
+        i += 7;
+        if (bytes[i++] != 0xa4) return false;
+        for (int f = 0; f < 4; ++f) {
+            const size_t nl = strlen(names[f]);
+            if (i + 1 + nl + 1 > len || bytes[i] != (0x60 | nl) || memcmp(bytes + i + 1, names[f], nl) != 0) return false;
+            i += 1 + nl;
+            const uint32_t b = bytes[i];
+            const int arg = cbor_item_len(b) - 1;
+            if ((b >> 5) != 0 || b > 0x1b || i + 1 + arg > len) return false;
+            uint64_t v = b < 24 ? b : 0;
+            for (int k = 0; k < arg; ++k) v = (v << 8) | bytes[i + 1 + k];
+            if (v > 0x7fffffffu) return false;
+            cfg[f] = (int)v;
+            i += 1 + arg;
+        }
+        return i == len;
+    }
+    return false;
+}
+
+}  // namespace
+
+zr_status kv_cbor_decode_device(zr_context* ctx, const uint8_t* bytes, size_t len, int layers, int rows, int cols,
+                                long long base_position, float* d_k, float* d_v, bool* taken) {
+    *taken = false;
+    int cfg[4];
+    if ((long long)rows * cols < kTokMinArray || len > (1ull << 40) || !tail_config(bytes, len, cfg)) return ZR_OK;
+    const KvCborLayout lay = kv_cbor_layout(layers, rows, cols, base_position, cfg);
+    const int arrays = 2 * layers;
+    if (len < lay.bytes.size() || memcmp(bytes, lay.bytes.data(), lay.len[0]) != 0) return ZR_OK;
+    const unsigned long long n = (unsigned long long)rows * cols;
+    const int blocks = (int)((len + kTokBlock - 1) / kTokBlock), groups = (blocks + 1023) / 1024;
+    // the bytes, then the passes' arrays; short of memory the strict reader takes the document
+    const size_t doc_bytes = (size_t)blocks * kTokBlock + 16;
+    const size_t threads = (size_t)blocks * kTokThreads;
+    const size_t words = threads + 2 * (size_t)blocks + 2 * (size_t)groups + 1 + 1 + 2 * (size_t)arrays;
+    const size_t need = words * 8 + 8 * (size_t)blocks + threads;
+    auto grow = [&](void** p, size_t* have, size_t want) {
+        if (*have >= want) return true;
+        if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+        *have = 0;
+        if (hipMalloc(p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            *p = nullptr;
+            return false;
+        }
+        *have = want;
+        return true;
+    };
+    if (!grow(&ctx->cbor_out, &ctx->cbor_out_bytes, doc_bytes) || !grow(&ctx->cbor_ws, &ctx->cbor_ws_bytes, need))
+        return ZR_OK;
+    TokArgs a;
+    a.doc = (const uint8_t*)ctx->cbor_out;
+    a.len = len;
+    a.blocks = blocks;
+    a.fn = (unsigned long long*)ctx->cbor_ws;
+    a.block_fn = a.fn + threads;
+    a.off = a.block_fn + blocks;
+    unsigned long long* group_tot = a.off + blocks;
+    a.group_off = group_tot + groups;
+    a.others = a.group_off + groups + 1;  // (read back together: floats, others, starts, ends)
+    a.starts = a.others + 1;
+    a.ends = a.starts + arrays;
+    a.entry = (uint32_t*)(a.ends + arrays);
+    a.block_floats = a.entry + blocks;
+    a.thread_floats = (uint8_t*)(a.block_floats + blocks);
+    a.arrays = arrays;
+    a.n = n;
+    a.k = d_k;
+    a.v = d_v;
+    ZR_HIP(ctx, hipMemcpyAsync(ctx->cbor_out, bytes, len, hipMemcpyDefault, ctx->stream));
+    hipEvent_t ev;
+    timing_mark_begin(ctx, kClassKvCbor, &ev);
+    hipLaunchKernelGGL(cbor_map_kernel, dim3(blocks), dim3(kTokThreads), 0, ctx->stream, a);
+    ZR_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(cbor_entry_kernel, dim3(1), dim3(1024), 0, ctx->stream, a);
+    ZR_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(cbor_tally_kernel, dim3(blocks), dim3(kTokThreads), 0, ctx->stream, a);
+    ZR_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(cbor_scan_groups_kernel, dim3(groups), dim3(1024), 0, ctx->stream, a.block_floats, blocks, a.off,
+                       group_tot);
+    ZR_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(cbor_scan_top_kernel, dim3(1), dim3(1024), 0, ctx->stream, group_tot, groups, a.group_off);
+    ZR_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(cbor_read_kernel, dim3(blocks), dim3(kTokThreads), 0, ctx->stream, a);
+    ZR_LAUNCH_CHECK(ctx);
+    timing_mark_end(ctx, kClassKvCbor, ev);
+    std::vector<unsigned long long> got(2 + 2 * (size_t)arrays);
+    ZR_HIP(ctx, hipMemcpyAsync(got.data(), a.group_off + groups, got.size() * 8, hipMemcpyDeviceToHost, ctx->stream));
+    ZR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    unsigned long long others = 0;
+    for (int i = 0; i <= arrays; ++i)
+        for (uint32_t p = 0; p < lay.len[i]; p += cbor_item_len(lay.bytes[lay.off[i] + p])) ++others;
+    if (got[0] != n * arrays || got[1] != others) return ZR_OK;
+    const unsigned long long *starts = got.data() + 2, *ends = starts + arrays;
+    for (int i = 0; i <= arrays; ++i) {  // gap i: before array i, after the last one
+        const unsigned long long g0 = i ? ends[i - 1] : 0, g1 = i < arrays ? starts[i] : (unsigned long long)len;
+        if (g0 > g1 || g1 > len || g1 - g0 != lay.len[i] || memcmp(bytes + g0, lay.bytes.data() + lay.off[i], lay.len[i]))
+            return ZR_OK;
+    }
+    *taken = true;
     return ZR_OK;
 }
 

@@ -243,9 +243,9 @@ struct zr_context {
     // would synchronise the device)
     hipStream_t d2h_stream = nullptr, h2d_stream = nullptr;
     std::vector<std::pair<float*, size_t>> xfer_free;
-    void* cbor_ws = nullptr;        // KV snapshot encoder: chunk sizes / offsets / header tables
+    void* cbor_ws = nullptr;        // KV snapshot encoder / decoder: chunk sizes, offsets, header tables, item maps
     size_t cbor_ws_bytes = 0;
-    void* cbor_out = nullptr;       // KV snapshot encoder: the document on the device
+    void* cbor_out = nullptr;       // KV snapshot encoder / decoder: the document on the device
     size_t cbor_out_bytes = 0;
     void* sample_ws = nullptr;      // stochastic sampling: per-row parameters
     size_t sample_ws_bytes = 0;
@@ -472,5 +472,14 @@ struct KvCborDoc {
     std::vector<float> k, v;          // [layers][rows][cols]
 };
 bool kv_cbor_decode(const uint8_t* bytes, size_t len, KvCborDoc* doc, std::string* err);
+// The rows of a document in the encoder's own form (these layers, rows, cols
+// and base position) decoded on the device into d_k / d_v [layers][rows][cols].
+// *taken = false (with ZR_OK) for any other document: kv_cbor_decode's.
+zr_status kv_cbor_decode_device(zr_context* ctx, const uint8_t* bytes, size_t len, int layers, int rows, int cols,
+                                long long base_position, float* d_k, float* d_v, bool* taken);
+// The K / V staging of a window ([layers][rows][kv_cols] K, then V, then room
+// for its page table), and the scatter of rows that are already in it.
+zr_status kv_stage_rows(zr_context* ctx, int n_rows, float** d_k, float** d_v);
+zr_status kv_scatter_staged(zr_context* ctx, const int* block_table, int n_pages, int first_offset, int n_rows);
 
 }  // namespace zr
