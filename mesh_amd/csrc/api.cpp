@@ -255,12 +255,20 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     st->h_items.clear();
     st->h_pblocks.clear();
     st->h_psplits.clear();
-    // sequences with >= 128 / G rows (prefill chunks) go to the prefill kernel
-    // as blocks of 128 / G rows (bf16 pools, G dividing 32)
+    // sequences with >= 128 / G rows (prefill chunks) go to the prefill kernels
+    // as blocks of 128 / G rows (G dividing 32)
     int prows = 0;
-    if (!ctx->plain_kv && ctx->desc.kv_dtype == ZR_DTYPE_BF16 && G <= 32 && 32 % G == 0) prows = 128 / G;
+    if (!ctx->plain_kv && G <= 32 && 32 % G == 0) prows = 128 / G;
     if (const char* env = getenv("ZR_ATTN_PREFILL"))
         if (atoi(env) == 0) prows = 0;
+    // ... from f32 pools where (row, q head) columns x visible keys are worth
+    // the blocks' fixed cost (append + attention of one chunk, decode tiles
+    // against blocks, us; 32 q / 4 kv heads of 64: 16 rows 31 / 33, 16 rows on
+    // 700 38 / 42, 128 rows 36 / 36, 64 rows on 1500 46 / 44, 32 rows on 6000
+    // 57 / 53, 128 on 6000 116 / 64; 32 / 8 heads of 128: 128 rows 42 / 43, 64
+    // on 1500 69 / 53, 1000 on 6000 1212 / 381)
+    const bool f32_kv = ctx->desc.kv_dtype == ZR_DTYPE_F32;
+    constexpr long kPrefillF32Work = 200000;
     if (ctx->plain_kv && ctx->head_dim % 4 == 0) {
         st->plain = plain_attention_plan(ctx->head_dim, ctx->local_kv_heads, G, mb->q_len, S);
         const long width = 16L * st->plain.ct;
@@ -280,7 +288,7 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     long total_pages = 0, total_ktiles = 0;
     for (int s = 0; s < S && qpt > 0; ++s) {
         const int ql = mb->q_len[s], kb = mb->kv_before[s], fo = mb->first_offset[s];
-        if (prows && ql >= prows) {
+        if (prows && ql >= prows && (!f32_kv || (long)ql * G * (kb + ql / 2) >= kPrefillF32Work)) {
             for (int r0 = 0; r0 < ql; r0 += prows) {
                 const int nr = std::min(prows, ql - r0);
                 const int last_visible = kb + r0 + nr - 1;
@@ -344,8 +352,13 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     // partials per 16-column group (16 / G rows x G heads, the decode tiles'
     // layout), one item per (group, split) after the decode items, and its
     // groups join the merge list as tiles.
+    // f32 blocks split down to 8 tiles, at most 16 splits (what the merge
+    // combines in one round trip): 64 rows on 1500, 32 / 8 heads of 128: 53 us
+    // with 8-tile splits, 62 with 16, 75 with 32; 32 rows on 6000: 71 / 64 / 84.
     const long slots = 512 / kh;
-    int tps = (int)std::max<long>(16 * kh, (total_ktiles * ctx->local_kv_heads + slots - 1) / slots);
+    int tps = (int)std::max<long>(f32_kv ? 8 : 16 * kh, (total_ktiles * ctx->local_kv_heads + slots - 1) / slots);
+    if (f32_kv)
+        for (const int4& b : pblk) tps = std::max(tps, ((b.w + 1) / 2 + 15) / 16);
     if ((long)pblk.size() * ctx->local_kv_heads >= slots) tps = 1 << 30;
     if (const char* env = getenv("ZR_ATTN_PREFILL_TILES_PER_SPLIT")) tps = std::max(1, atoi(env));
     if (G > 16) tps = 1 << 30;  // a 16-column group must hold whole rows

@@ -7,9 +7,9 @@
 //   [0, prefix + r].
 //
 // Two kernels share one launch slot: sequences with at least 128 / G query
-// rows in a bf16 pool (prefill chunks) run paged_prefill_attention_kernel
-// (further below); every other row (decode rows, short chunks, f32 pools)
-// runs paged_attention_kernel.
+// rows (prefill chunks) run paged_prefill_attention_kernel or, from f32 pools,
+// paged_prefill_attention_f32_kernel (further below); every other row (decode
+// rows, short chunks) runs paged_attention_kernel.
 //
 // Work decomposition.  A workgroup is one wavefront (64 lanes).  It owns one
 // kv head of one "tile" and a contiguous range of KV pages (a split):
@@ -556,8 +556,8 @@ __global__ __launch_bounds__(64) void paged_attention_kernel(AttnArgs a) {
 }
 
 // ------------------------------------------------------------ prefill blocks
-// Sequences with at least 128 / G query rows (prefill chunks) run here, bf16
-// pools only.  A workgroup of 4 waves owns one kv head of one block of
+// Sequences with at least 128 / G query rows (prefill chunks) run here (bf16
+// pools; f32 pools in the kernel after it).  A workgroup of 4 waves owns one kv head of one block of
 // 128 / G query rows: 128 columns = (row, q head of the kv head) pairs, 32
 // per wave.  Every 32-key tile (two pages) of the block's visible window is
 // copied once into an LDS ring with global_load_lds (the pool's page layout,
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(64) void paged_attention_kernel(AttnArgs a) {
 struct PrefillArgs {
     const float* q;          // [T, q_cols]
     int q_cols;
-    const uint16_t* pool;    // layer base of the pool (bf16)
+    const void* pool;        // layer base of the pool
     size_t page_elems;
     int stride;              // block table row stride (the table is a kernel argument)
     const int* first_offset;
@@ -608,241 +608,82 @@ __device__ inline float pair_sum(float x) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-template <int D, int STAGES, int KH>
-__global__ __launch_bounds__(256 * KH, 2 / KH) void paged_prefill_attention_kernel(PrefillArgs a,
-                                                                               const int* __restrict__ block_tables) {
-    constexpr int NW = 4;            // column waves (32 columns each)
-    constexpr int CHUNKS = 8 * D;   // 16 B chunks per tile: 2 pages x (K, V) x 16 rows x D bf16
-    constexpr int VM = D / 32;      // global_load_lds per wave per stage (1 KiB each)
-    static_assert(CHUNKS == NW * VM * 64, "stage copy split");
-    static_assert(KH == 1 || KH == 2, "key halves");
-    // a stage holds KH consecutive key tiles, tile h for the waves of half h
-    __shared__ bf16x8 lds[STAGES][KH][CHUNKS];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int half = wave / NW, wq = wave - half * NW;  // key half, column wave
-    // block-uniform values in scalar registers
-    const int rank = __builtin_amdgcn_readfirstlane(blockIdx.x / a.kv_heads);
-    const int kvh = blockIdx.x - rank * a.kv_heads;
-    const int4 blk = a.blocks[rank];
-    const int4 spl = a.splits[rank];
-    const int seq = __builtin_amdgcn_readfirstlane(blk.x), r0 = __builtin_amdgcn_readfirstlane(blk.y);
-    const int nrows = __builtin_amdgcn_readfirstlane(blk.z), npages = __builtin_amdgcn_readfirstlane(blk.w);
-    const int kt0 = __builtin_amdgcn_readfirstlane(spl.x), kt1 = __builtin_amdgcn_readfirstlane(spl.y);
-    const int h = lane >> 5;
-    const int col = lane & 31;
-    const int rpw = 32 / a.G;  // query rows per column wave
-    const int rloc = wq * rpw + col / a.G, g = col - (col / a.G) * a.G;
-    const bool valid = rloc < nrows;
-    const int kvb = __builtin_amdgcn_readfirstlane(a.kv_before[seq]);
-    const int foff = __builtin_amdgcn_readfirstlane(a.first_offset[seq]);
-    const int jmax = kvb + r0 + (valid ? rloc : 0);  // last visible logical key of this column
-    const int grow = __builtin_amdgcn_readfirstlane(a.cu_q[seq]) + r0 + (valid ? rloc : 0);
-
-    const uint16_t* pool = a.pool;
-    // (a restrict kernel argument: nothing here writes it, so its reads are scalar loads)
-    const int* bt = block_tables + (size_t)seq * a.stride;
-    const size_t kv_tile = (size_t)kPageRows * D;
-    const size_t v_block = (size_t)a.kv_heads * kv_tile;
-    // Key tiles [kt0, kt1) go in steps of KH: step p holds tile kt0 + KH p + h
-    // for the waves of half h.  A half stages its own tile of each step into
-    // ring slot `slot` from the pool pages of the tile's two pages (pg0, pg1):
-    // chunk group f = i NW + wq is (page pp, K or V, 1 KiB group); a page past
-    // the window's end repeats the last page (its keys are masked, and a tile
-    // past kt1 is copied the same way and skipped), so every wave issues VM
-    // copies per stage.  The page ids are read a step ahead (tile_pages), so
-    // no scalar load waits in front of a stage's copies.
-    auto tile_pages = [&](int kt, int& pg0, int& pg1) {
-        pg0 = __builtin_amdgcn_readfirstlane(bt[min(2 * kt, npages - 1)]);
-        pg1 = __builtin_amdgcn_readfirstlane(bt[min(2 * kt + 1, npages - 1)]);
-    };
-    // Copies are buffer loads into LDS over one page: the page's base in the
-    // (scalar) buffer descriptor, the lane's 16 B as the vector offset, the
-    // K / V block, kv head and 1 KiB group as a scalar offset.
-    const uint32_t page_bytes = (uint32_t)(a.page_elems * 2);
-    const int voff = lane * 16;
-    auto issue = [&](int slot, int pg0, int pg1) {
-        const __amdgpu_buffer_rsrc_t r0 =
-            __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)pg0 * a.page_elems), 0, page_bytes, 0x00020000);
-        const __amdgpu_buffer_rsrc_t r1 =
-            __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)pg1 * a.page_elems), 0, page_bytes, 0x00020000);
+// Q^T fragments (B operand) of a column: lane holds Q[col][16 ks + 8 h + j]
+// log2(e) / sqrt(d) as hi + lo (scores come out in log2 units).
+template <int D>
+__device__ __forceinline__ void prefill_load_q(const PrefillArgs& a, size_t at, bool valid, bf16x8 (&qh)[D / 16],
+                                               bf16x8 (&ql)[D / 16]) {
+    const float* qp = a.q + at;
 #pragma unroll
-        for (int i = 0; i < VM; ++i) {
-            const int f = i * NW + wq;
-            const int pp = f / (2 * VM), kv = (f / VM) & 1, grp = f % VM;
-            const int soff = (int)(((kv ? v_block : 0) + (size_t)kvh * kv_tile) * 2) + grp * 1024;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(pp ? r1 : r0, (lds_void*)&lds[slot][half][f * 64], 16, voff, soff,
-                                                     0, 0);
+    for (int ks = 0; ks < D / 16; ++ks) {
+        float x[8];
+        const f32x4 x0 = valid ? *(const f32x4*)(qp + 16 * ks) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const f32x4 x1 = valid ? *(const f32x4*)(qp + 16 * ks + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[j] = x0[j] * a.scale_log2;
+            x[4 + j] = x1[j] * a.scale_log2;
         }
-    };
-
-    f32x16 o[D / 32];
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
-    float m = -INFINITY, lsum = 0.0f;
-
-    // a tile needs the causal mask only if it may hold a key before the
-    // window (first_offset) or after the block's first row's last visible key
-    const int ntiles = kt1 - kt0;
-    const int nsteps = (ntiles + KH - 1) / KH;
-    const int jfree = kvb + r0;  // keys <= jfree are visible to every row of the block
-    int npg0 = 0, npg1 = 0;  // pool pages of this half's tile of the next step to stage
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
-        if (s < nsteps) {
-            tile_pages(kt0 + KH * s + half, npg0, npg1);
-            issue(s, npg0, npg1);
-        }
-    tile_pages(kt0 + KH * (STAGES - 1) + half, npg0, npg1);
-    // Q^T fragments (B operand): lane holds Q[col][16 ks + 8 h + j] * log2(e) / sqrt(d)
-    // as hi + lo (scores come out in log2 units).  Loaded after the first
-    // stages' copies are issued, so both latencies overlap.
-    bf16x8 qh[D / 16], ql[D / 16];
-    {
-        const float* qp = a.q + (size_t)grow * a.q_cols + (size_t)(kvh * a.G + g) * D + 8 * h;
-#pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) {
-            float x[8];
-            const f32x4 x0 = valid ? *(const f32x4*)(qp + 16 * ks) : f32x4{0.f, 0.f, 0.f, 0.f};
-            const f32x4 x1 = valid ? *(const f32x4*)(qp + 16 * ks + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                x[j] = x0[j] * a.scale_log2;
-                x[4 + j] = x1[j] * a.scale_log2;
-            }
-            qh[ks] = to_bf16x8(x, false);
-            ql[ks] = to_bf16x8(x, true);
-        }
+        qh[ks] = to_bf16x8(x, false);
+        ql[ks] = to_bf16x8(x, true);
     }
-    // One tile of a half in two parts.  phase_s: the tile's LDS fragments,
-    // read in two batches ahead of their consumers (K before the S = K Q^T
-    // MFMAs, V before the softmax, whose VALU work covers their return), and
-    // S.  phase_p: the causal mask where needed, the online softmax step and
-    // O += V^T P, on registers only.
-    f32x16 s;
-    bf16x8 vfr[2][D / 32];
-    int s_it = 0;        // key tile held in s / vfr
-    bool s_act = false;  // ... and whether it is one of the block's tiles
-    auto phase_s = [&](int t) {
-        s_it = kt0 + KH * t + half;
-        s_act = KH == 1 || s_it < kt1;
-        if (!s_act) {
-            // (s and vfr are written on every path, so the previous tile's
-            // values are not kept alive through this one)
+}
+
+// Scores of keys a column does not see: element i is logical key jbase + 8 (i / 4) + i % 4.
+__device__ __forceinline__ void prefill_mask(f32x16& s, int jbase, int jmax) {
+    asm volatile("" ::: "memory");
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-#pragma unroll
-            for (int ks2 = 0; ks2 < 2; ++ks2)
-#pragma unroll
-                for (int db = 0; db < D / 32; ++db) vfr[ks2][db] = bf16x8{};
-            return;
-        }
-        const bf16x8* st = lds[t % STAGES][half];
-        const int kbase = ((lane >> 4) & 1) * 2 * (2 * D) + (lane & 15);  // page pp = (l % 32) / 16, row l % 16
-        bf16x8 kf[D / 16];
-#pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) kf[ks] = st[kbase + (2 * ks + h) * 16];
-        __builtin_amdgcn_sched_barrier(0);  // the K reads stay ahead of the MFMAs
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) {
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qh[ks], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], ql[ks], s, 0, 0, 0);
-        }
-        const bf16x4* sv = (const bf16x4*)st;
-#pragma unroll
-        for (int ks2 = 0; ks2 < 2; ++ks2) {
-            const int vbase = (2 * ks2 + 1) * 4 * D;  // 8-byte units of page ks2's V block
-#pragma unroll
-            for (int db = 0; db < D / 32; ++db) {
-                // unit of (rows 4 q .. 4 q + 3, dim d): ((d / 32 * 4 + q) * 16 + d % 16) * 2 + d / 16 % 2
-                const int u = ((db * 4 + h) * 16 + (lane & 15)) * 2 + ((lane >> 4) & 1);
-                const bf16x4 v0 = sv[vbase + u], v1 = sv[vbase + u + 2 * 16 * 2];
-                vfr[ks2][db] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // the V reads go out before the softmax
-    };
-    auto phase_p = [&]() {
-        if (!s_act) return;
-        const int it = s_it;
-        // the causal mask only on tiles that can hold a key before the window
-        // or past the block's first row (a uniform branch, kept out of the
-        // common path)
-        if (it * 32 - foff < 0 || it * 32 + 31 - foff > jfree) {
-            asm volatile("" ::: "memory");
-            const int jbase = it * 32 + 4 * h - foff;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int j = jbase + 8 * (i >> 2) + (i & 3);
-                if (j < 0 || j > jmax) s[i] = -INFINITY;
-            }
-        }
-        float tmax = s[0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
-        tmax = pair_max(tmax);
-        // Lazy rescale: a column keeps its running max m until a tile's max
-        // exceeds it by more than 8 (log2 units), so P <= 2^8 and O and l are
-        // rescaled only when some column of the wave moves that far (the first
-        // tile with a visible key, then rarely).  The result is the same
-        // softmax: O and l share the scale.
-        if (__any(tmax > m + 8.0f)) {
-            // only the lanes whose max moves rescale (alpha 0 while m = -inf);
-            // the others keep alpha = 1 exactly, also a column with no visible
-            // key yet (m = -inf, where m - m would be NaN)
-            const bool up = tmax > m + 8.0f;
-            const float alpha = up ? __builtin_amdgcn_exp2f(m - tmax) : 1.0f;
-            if (up) m = tmax;
-            lsum *= alpha;
-#pragma unroll
-            for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
-        }
-        const float m_use = m == -INFINITY ? 0.0f : m;
-        float pr[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            pr[i] = __builtin_amdgcn_exp2f(s[i] - m_use);
-            lsum += pr[i];
-        }
-        // O += V^T P over the tile's two pages (k-steps ks2)
-#pragma unroll
-        for (int ks2 = 0; ks2 < 2; ++ks2) {
-            bf16x8 ph, pl;
-            split_bf16x8(pr + 8 * ks2, ph, pl);
-#pragma unroll
-            for (int db = 0; db < D / 32; ++db) {
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[ks2][db], ph, o[db], 0, 0, 0);
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[ks2][db], pl, o[db], 0, 0, 0);
-            }
-        }
-    };
-    // the page ids of the step after the one just staged, read once this
-    // step's LDS reads have been issued and waited for (scalar loads return
-    // out of order: one in flight would turn every LDS wait into a full
-    // drain); the next ring barrier waits for them
-    auto prefetch_pages = [&](int t) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (t + STAGES - 1 < nsteps) tile_pages(kt0 + KH * (t + STAGES) + half, npg0, npg1);
-    };
-    // One loop for both forms: with KH = 2 each half takes every other key
-    // tile (kt0 + 2 t + half) of the block.  (A second barrier per step that
-    // offset the halves into MFMA-bound and VALU-bound phases measured slower
-    // once the copies were descriptor-based: mixed 2108-row microbatch, prefill
-    // kernel 90.9-91.1 against 87.4-87.7 us per layer without it.)
-    for (int t = 0; t < nsteps; ++t) {
-        ring_wait<VM, STAGES - 2>(min(STAGES - 2, nsteps - 1 - t));
-        if (t + STAGES - 1 < nsteps) issue((t + STAGES - 1) % STAGES, npg0, npg1);
-        phase_s(t);
-        phase_p();
-        prefetch_pages(t);
+    for (int i = 0; i < 16; ++i) {
+        const int j = jbase + 8 * (i >> 2) + (i & 3);
+        if (j < 0 || j > jmax) s[i] = -INFINITY;
     }
+}
+
+// One online softmax step over a tile's scores: pr = 2^(s - m), l and O
+// rescaled where m moves.
+template <int D>
+__device__ __forceinline__ void prefill_softmax(const f32x16& s, f32x16 (&o)[D / 32], float& m, float& lsum,
+                                                float (&pr)[16]) {
+    float tmax = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
+    tmax = pair_max(tmax);
+    // Lazy rescale: a column keeps its running max m until a tile's max
+    // exceeds it by more than 8 (log2 units), so P <= 2^8 and O and l are
+    // rescaled only when some column of the wave moves that far (the first
+    // tile with a visible key, then rarely).  The result is the same
+    // softmax: O and l share the scale.
+    if (__any(tmax > m + 8.0f)) {
+        // only the lanes whose max moves rescale (alpha 0 while m = -inf);
+        // the others keep alpha = 1 exactly, also a column with no visible
+        // key yet (m = -inf, where m - m would be NaN)
+        const bool up = tmax > m + 8.0f;
+        const float alpha = up ? __builtin_amdgcn_exp2f(m - tmax) : 1.0f;
+        if (up) m = tmax;
+        lsum *= alpha;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+    }
+    const float m_use = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        pr[i] = __builtin_amdgcn_exp2f(s[i] - m_use);
+        lsum += pr[i];
+    }
+}
+
+// The end of a prefill block: with KH = 2 the halves' (m, l, O) of each column
+// meet in `ring` (the block's LDS ring, prefill_combine_bytes of it), then the
+// columns go out as one split's partials or as the final rows.
+constexpr size_t prefill_combine_bytes(int D) { return (size_t)4 * (2 + 16 * (D / 32)) * 64 * 4; }
+
+template <int D, int KH>
+__device__ __forceinline__ void prefill_finish(const PrefillArgs& a, const int4& spl, f32x16 (&o)[D / 32], float m,
+                                               float lsum, float* ring, int half, int wq, int lane, int kvh, int g,
+                                               int grow, bool valid) {
+    const int h = lane >> 5, col = lane & 31;
     lsum = pair_sum(lsum);
     if constexpr (KH == 2) {
         // The halves' (m, l, O) of each column meet in LDS (the ring is free:
@@ -850,8 +691,7 @@ __global__ __launch_bounds__(256 * KH, 2 / KH) void paged_prefill_attention_kern
         // writes, half 0 rescales both to the larger m and adds.  A half with
         // no visible key in its tiles (m = -inf, l = 0, O = 0) gets weight 0.
         constexpr int CW = 2 + 16 * (D / 32);  // floats per column lane
-        static_assert((size_t)NW * CW * 64 * 4 <= sizeof(lds), "combine buffer");
-        float* cmb = (float*)&lds[0][0][0] + (size_t)wq * CW * 64 + lane;  // [wq][j][lane]
+        float* cmb = ring + (size_t)wq * CW * 64 + lane;  // [wq][j][lane]
         __syncthreads();
         if (half == 1) {
             cmb[0] = m;
@@ -930,6 +770,412 @@ __global__ __launch_bounds__(256 * KH, 2 / KH) void paged_prefill_attention_kern
                              o[db][4 * i4 + 3] * inv};
             *(f32x4*)(a.out_f32 + (size_t)grow * a.q_cols + ocol0 + d) = v;
         }
+}
+
+template <int D, int STAGES, int KH>
+__global__ __launch_bounds__(256 * KH, 2 / KH) void paged_prefill_attention_kernel(PrefillArgs a,
+                                                                               const int* __restrict__ block_tables) {
+    constexpr int NW = 4;            // column waves (32 columns each)
+    constexpr int CHUNKS = 8 * D;   // 16 B chunks per tile: 2 pages x (K, V) x 16 rows x D bf16
+    constexpr int VM = D / 32;      // global_load_lds per wave per stage (1 KiB each)
+    static_assert(CHUNKS == NW * VM * 64, "stage copy split");
+    static_assert(KH == 1 || KH == 2, "key halves");
+    // a stage holds KH consecutive key tiles, tile h for the waves of half h
+    __shared__ bf16x8 lds[STAGES][KH][CHUNKS];
+    static_assert(KH == 1 || prefill_combine_bytes(D) <= sizeof(lds), "combine buffer");
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = wave / NW, wq = wave - half * NW;  // key half, column wave
+    // block-uniform values in scalar registers
+    const int rank = __builtin_amdgcn_readfirstlane(blockIdx.x / a.kv_heads);
+    const int kvh = blockIdx.x - rank * a.kv_heads;
+    const int4 blk = a.blocks[rank];
+    const int4 spl = a.splits[rank];
+    const int seq = __builtin_amdgcn_readfirstlane(blk.x), r0 = __builtin_amdgcn_readfirstlane(blk.y);
+    const int nrows = __builtin_amdgcn_readfirstlane(blk.z), npages = __builtin_amdgcn_readfirstlane(blk.w);
+    const int kt0 = __builtin_amdgcn_readfirstlane(spl.x), kt1 = __builtin_amdgcn_readfirstlane(spl.y);
+    const int h = lane >> 5;
+    const int col = lane & 31;
+    const int rpw = 32 / a.G;  // query rows per column wave
+    const int rloc = wq * rpw + col / a.G, g = col - (col / a.G) * a.G;
+    const bool valid = rloc < nrows;
+    const int kvb = __builtin_amdgcn_readfirstlane(a.kv_before[seq]);
+    const int foff = __builtin_amdgcn_readfirstlane(a.first_offset[seq]);
+    const int jmax = kvb + r0 + (valid ? rloc : 0);  // last visible logical key of this column
+    const int grow = __builtin_amdgcn_readfirstlane(a.cu_q[seq]) + r0 + (valid ? rloc : 0);
+
+    const uint16_t* pool = (const uint16_t*)a.pool;
+    // (a restrict kernel argument: nothing here writes it, so its reads are scalar loads)
+    const int* bt = block_tables + (size_t)seq * a.stride;
+    const size_t kv_tile = (size_t)kPageRows * D;
+    const size_t v_block = (size_t)a.kv_heads * kv_tile;
+    // Key tiles [kt0, kt1) go in steps of KH: step p holds tile kt0 + KH p + h
+    // for the waves of half h.  A half stages its own tile of each step into
+    // ring slot `slot` from the pool pages of the tile's two pages (pg0, pg1):
+    // chunk group f = i NW + wq is (page pp, K or V, 1 KiB group); a page past
+    // the window's end repeats the last page (its keys are masked, and a tile
+    // past kt1 is copied the same way and skipped), so every wave issues VM
+    // copies per stage.  The page ids are read a step ahead (tile_pages), so
+    // no scalar load waits in front of a stage's copies.
+    auto tile_pages = [&](int kt, int& pg0, int& pg1) {
+        pg0 = __builtin_amdgcn_readfirstlane(bt[min(2 * kt, npages - 1)]);
+        pg1 = __builtin_amdgcn_readfirstlane(bt[min(2 * kt + 1, npages - 1)]);
+    };
+    // Copies are buffer loads into LDS over one page: the page's base in the
+    // (scalar) buffer descriptor, the lane's 16 B as the vector offset, the
+    // K / V block, kv head and 1 KiB group as a scalar offset.
+    const uint32_t page_bytes = (uint32_t)(a.page_elems * 2);
+    const int voff = lane * 16;
+    auto issue = [&](int slot, int pg0, int pg1) {
+        const __amdgpu_buffer_rsrc_t r0 =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)pg0 * a.page_elems), 0, page_bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t r1 =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)pg1 * a.page_elems), 0, page_bytes, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < VM; ++i) {
+            const int f = i * NW + wq;
+            const int pp = f / (2 * VM), kv = (f / VM) & 1, grp = f % VM;
+            const int soff = (int)(((kv ? v_block : 0) + (size_t)kvh * kv_tile) * 2) + grp * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(pp ? r1 : r0, (lds_void*)&lds[slot][half][f * 64], 16, voff, soff,
+                                                     0, 0);
+        }
+    };
+
+    f32x16 o[D / 32];
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
+    float m = -INFINITY, lsum = 0.0f;
+
+    // a tile needs the causal mask only if it may hold a key before the
+    // window (first_offset) or after the block's first row's last visible key
+    const int ntiles = kt1 - kt0;
+    const int nsteps = (ntiles + KH - 1) / KH;
+    const int jfree = kvb + r0;  // keys <= jfree are visible to every row of the block
+    int npg0 = 0, npg1 = 0;  // pool pages of this half's tile of the next step to stage
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+        if (s < nsteps) {
+            tile_pages(kt0 + KH * s + half, npg0, npg1);
+            issue(s, npg0, npg1);
+        }
+    tile_pages(kt0 + KH * (STAGES - 1) + half, npg0, npg1);
+    // Q^T fragments (B operand): lane holds Q[col][16 ks + 8 h + j] * log2(e) / sqrt(d)
+    // as hi + lo (scores come out in log2 units).  Loaded after the first
+    // stages' copies are issued, so both latencies overlap.
+    bf16x8 qh[D / 16], ql[D / 16];
+    prefill_load_q<D>(a, (size_t)grow * a.q_cols + (size_t)(kvh * a.G + g) * D + 8 * h, valid, qh, ql);
+    // One tile of a half in two parts.  phase_s: the tile's LDS fragments,
+    // read in two batches ahead of their consumers (K before the S = K Q^T
+    // MFMAs, V before the softmax, whose VALU work covers their return), and
+    // S.  phase_p: the causal mask where needed, the online softmax step and
+    // O += V^T P, on registers only.
+    f32x16 s;
+    bf16x8 vfr[2][D / 32];
+    int s_it = 0;        // key tile held in s / vfr
+    bool s_act = false;  // ... and whether it is one of the block's tiles
+    auto phase_s = [&](int t) {
+        s_it = kt0 + KH * t + half;
+        s_act = KH == 1 || s_it < kt1;
+        if (!s_act) {
+            // (s and vfr are written on every path, so the previous tile's
+            // values are not kept alive through this one)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+            for (int ks2 = 0; ks2 < 2; ++ks2)
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) vfr[ks2][db] = bf16x8{};
+            return;
+        }
+        const bf16x8* st = lds[t % STAGES][half];
+        const int kbase = ((lane >> 4) & 1) * 2 * (2 * D) + (lane & 15);  // page pp = (l % 32) / 16, row l % 16
+        bf16x8 kf[D / 16];
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) kf[ks] = st[kbase + (2 * ks + h) * 16];
+        __builtin_amdgcn_sched_barrier(0);  // the K reads stay ahead of the MFMAs
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) {
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qh[ks], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], ql[ks], s, 0, 0, 0);
+        }
+        const bf16x4* sv = (const bf16x4*)st;
+#pragma unroll
+        for (int ks2 = 0; ks2 < 2; ++ks2) {
+            const int vbase = (2 * ks2 + 1) * 4 * D;  // 8-byte units of page ks2's V block
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) {
+                // unit of (rows 4 q .. 4 q + 3, dim d): ((d / 32 * 4 + q) * 16 + d % 16) * 2 + d / 16 % 2
+                const int u = ((db * 4 + h) * 16 + (lane & 15)) * 2 + ((lane >> 4) & 1);
+                const bf16x4 v0 = sv[vbase + u], v1 = sv[vbase + u + 2 * 16 * 2];
+                vfr[ks2][db] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the V reads go out before the softmax
+    };
+    auto phase_p = [&]() {
+        if (!s_act) return;
+        const int it = s_it;
+        // the causal mask only on tiles that can hold a key before the window
+        // or past the block's first row (a uniform branch, kept out of the
+        // common path)
+        if (it * 32 - foff < 0 || it * 32 + 31 - foff > jfree) prefill_mask(s, it * 32 + 4 * h - foff, jmax);
+        float pr[16];
+        prefill_softmax<D>(s, o, m, lsum, pr);
+        // O += V^T P over the tile's two pages (k-steps ks2)
+#pragma unroll
+        for (int ks2 = 0; ks2 < 2; ++ks2) {
+            bf16x8 ph, pl;
+            split_bf16x8(pr + 8 * ks2, ph, pl);
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) {
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[ks2][db], ph, o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[ks2][db], pl, o[db], 0, 0, 0);
+            }
+        }
+    };
+    // the page ids of the step after the one just staged, read once this
+    // step's LDS reads have been issued and waited for (scalar loads return
+    // out of order: one in flight would turn every LDS wait into a full
+    // drain); the next ring barrier waits for them
+    auto prefetch_pages = [&](int t) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + STAGES - 1 < nsteps) tile_pages(kt0 + KH * (t + STAGES) + half, npg0, npg1);
+    };
+    // One loop for both forms: with KH = 2 each half takes every other key
+    // tile (kt0 + 2 t + half) of the block.  (A second barrier per step that
+    // offset the halves into MFMA-bound and VALU-bound phases measured slower
+    // once the copies were descriptor-based: mixed 2108-row microbatch, prefill
+    // kernel 90.9-91.1 against 87.4-87.7 us per layer without it.)
+    for (int t = 0; t < nsteps; ++t) {
+        ring_wait<VM, STAGES - 2>(min(STAGES - 2, nsteps - 1 - t));
+        if (t + STAGES - 1 < nsteps) issue((t + STAGES - 1) % STAGES, npg0, npg1);
+        phase_s(t);
+        phase_p();
+        prefetch_pages(t);
+    }
+    prefill_finish<D, KH>(a, spl, o, m, lsum, (float*)&lds[0][0][0], half, wq, lane, kvh, g, grow, valid);
+}
+
+// The same blocks over f32 pools: K, V, Q and P each enter the MFMA as bf16
+// hi + lo (three products of each pair, as in paged_attention_kernel's f32
+// pages).  A tile is split once per workgroup: each wave of a half loads its
+// quarter of the next tile's f32 groups into registers a whole step ahead,
+// splits them and stores hi and lo planes in the LDS layout of a bf16 tile,
+// two slots deep, one barrier per step.  (The decode kernel read each page
+// once per 16 columns and split it again in every tile.)  The 997-row
+// TinyLlama prompt: 36 us per layer against 56 and a 6 us merge; one 1000-row
+// chunk on 6000 rows, 32 q / 8 kv heads of 128, append included: 381 us
+// against 1212.
+// Bound by the MFMAs: 48 of 32x32x16 per tile and wave at head_dim 128.
+template <int D, int KH>
+__global__ __launch_bounds__(256 * KH, 2 / KH) void paged_prefill_attention_f32_kernel(
+    PrefillArgs a, const int* __restrict__ block_tables) {
+    constexpr int NW = 4;          // column waves (32 columns each)
+    constexpr int CHUNKS = 8 * D;  // 16 B chunks per plane of a tile: 2 pages x (K, V) x 16 rows x D bf16
+    constexpr int VM = D / 32;     // 512-element groups per wave and tile
+    __shared__ bf16x8 lds[2][KH][2][CHUNKS];  // [slot][half][hi, lo]
+    static_assert(KH == 1 || prefill_combine_bytes(D) <= sizeof(lds), "combine buffer");
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = wave / NW, wq = wave - half * NW;
+    const int rank = __builtin_amdgcn_readfirstlane(blockIdx.x / a.kv_heads);
+    const int kvh = blockIdx.x - rank * a.kv_heads;
+    const int4 blk = a.blocks[rank];
+    const int4 spl = a.splits[rank];
+    const int seq = __builtin_amdgcn_readfirstlane(blk.x), r0 = __builtin_amdgcn_readfirstlane(blk.y);
+    const int nrows = __builtin_amdgcn_readfirstlane(blk.z), npages = __builtin_amdgcn_readfirstlane(blk.w);
+    const int kt0 = __builtin_amdgcn_readfirstlane(spl.x), kt1 = __builtin_amdgcn_readfirstlane(spl.y);
+    const int h = lane >> 5;
+    const int col = lane & 31;
+    const int rpw = 32 / a.G;
+    const int rloc = wq * rpw + col / a.G, g = col - (col / a.G) * a.G;
+    const bool valid = rloc < nrows;
+    const int kvb = __builtin_amdgcn_readfirstlane(a.kv_before[seq]);
+    const int foff = __builtin_amdgcn_readfirstlane(a.first_offset[seq]);
+    const int jmax = kvb + r0 + (valid ? rloc : 0);
+    const int grow = __builtin_amdgcn_readfirstlane(a.cu_q[seq]) + r0 + (valid ? rloc : 0);
+    const int* bt = block_tables + (size_t)seq * a.stride;
+    const size_t kv_tile = (size_t)kPageRows * D;
+    const size_t v_block = (size_t)a.kv_heads * kv_tile;
+    const float* pool = (const float*)a.pool + (size_t)kvh * kv_tile + 4 * lane;
+
+    auto tile_pages = [&](int kt, int& pg0, int& pg1) {
+        pg0 = __builtin_amdgcn_readfirstlane(bt[min(2 * kt, npages - 1)]);
+        pg1 = __builtin_amdgcn_readfirstlane(bt[min(2 * kt + 1, npages - 1)]);
+    };
+    f32x4 raw[VM][2];  // this wave's groups of the next tile (group f = 4 i + wq: page, K or V, 512-element run)
+    auto load_raw = [&](int pg0, int pg1) {
+#pragma unroll
+        for (int i = 0; i < VM; ++i) {
+            const int f = i * NW + wq;
+            const int pp = f / (2 * VM), kv = (f / VM) & 1, grp = f % VM;
+            const f32x4* src =
+                (const f32x4*)(pool + (size_t)(pp ? pg1 : pg0) * a.page_elems + (kv ? v_block : 0) + (size_t)grp * 512);
+            raw[i][0] = src[0];
+            raw[i][1] = src[kWave];
+        }
+    };
+    // Weights of keys a column does not see are 0, but 0 x inf is NaN: a V
+    // value that is not finite enters the product as 0, and the columns that
+    // see it are marked after the loop (rows of a page past or before the
+    // window, or of the chunk's later queries, then reach no one).
+    bool not_finite = false;
+    auto store_split = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < VM; ++i) {
+            const int f = i * NW + wq;
+            float x[8] = {raw[i][0][0], raw[i][0][1], raw[i][0][2], raw[i][0][3],
+                          raw[i][1][0], raw[i][1][1], raw[i][1][2], raw[i][1][3]};
+            if ((f / VM) & 1) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool bad = !__builtin_isfinite(x[j]);
+                    not_finite |= bad;
+                    x[j] = bad ? 0.0f : x[j];
+                }
+            }
+            bf16x8 hi, lo;
+            split_bf16x8(x, hi, lo);
+            lds[slot][half][0][f * 64 + lane] = hi;
+            lds[slot][half][1][f * 64 + lane] = lo;
+        }
+    };
+
+    f32x16 o[D / 32];
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
+    float m = -INFINITY, lsum = 0.0f;
+    const int ntiles = kt1 - kt0;
+    const int nsteps = (ntiles + KH - 1) / KH;
+    const int jfree = kvb + r0;
+    int pg0, pg1, npg0, npg1;
+    tile_pages(kt0 + half, pg0, pg1);
+    tile_pages(kt0 + KH + half, npg0, npg1);
+    load_raw(pg0, pg1);
+    bf16x8 qh[D / 16], ql[D / 16];
+    prefill_load_q<D>(a, (size_t)grow * a.q_cols + (size_t)(kvh * a.G + g) * D + 8 * h, valid, qh, ql);
+    store_split(0);
+    load_raw(npg0, npg1);
+    tile_pages(kt0 + 2 * KH + half, npg0, npg1);
+
+    // V^T fragments of a plane: two 8-byte runs of the page's V layout per 32 dims
+    auto v_frags = [&](const bf16x8* plane, bf16x8 (&v)[2][D / 32]) {
+        const bf16x4* sv = (const bf16x4*)plane;
+#pragma unroll
+        for (int ks2 = 0; ks2 < 2; ++ks2) {
+            const int vbase = (2 * ks2 + 1) * 4 * D;
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) {
+                const int u = ((db * 4 + h) * 16 + (lane & 15)) * 2 + ((lane >> 4) & 1);
+                const bf16x4 v0 = sv[vbase + u], v1 = sv[vbase + u + 2 * 16 * 2];
+                v[ks2][db] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        }
+    };
+
+    for (int t = 0; t < nsteps; ++t) {
+        ring_barrier<63>();  // slot t % 2 is written (LDS only: the next tile's loads stay in flight)
+        const int it = kt0 + KH * t + half;
+        if (KH == 1 || it < kt1) {
+            const bf16x8* hi = lds[t & 1][half][0];
+            const bf16x8* lo = lds[t & 1][half][1];
+            const int kbase = ((lane >> 4) & 1) * 2 * (2 * D) + (lane & 15);
+            f32x16 s;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {  // K in two batches of dims (registers)
+                bf16x8 kh[D / 32], kl[D / 32];
+#pragma unroll
+                for (int i = 0; i < D / 32; ++i) {
+                    const int ks = b * (D / 32) + i;
+                    kh[i] = hi[kbase + (2 * ks + h) * 16];
+                    kl[i] = lo[kbase + (2 * ks + h) * 16];
+                }
+#pragma unroll
+                for (int i = 0; i < D / 32; ++i) {
+                    const int ks = b * (D / 32) + i;
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh[i], qh[ks], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh[i], ql[ks], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kl[i], qh[ks], s, 0, 0, 0);
+                }
+            }
+            bf16x8 vf[2][D / 32];
+            v_frags(hi, vf);
+            __builtin_amdgcn_sched_barrier(0);  // the V reads go out before the softmax
+            const int j0 = it * 32 - foff;
+            if (j0 < 0 || j0 + 31 > jfree) prefill_mask(s, j0 + 4 * h, jmax);
+            float pr[16];
+            prefill_softmax<D>(s, o, m, lsum, pr);
+            bf16x8 ph[2], pl[2];
+            split_bf16x8(pr, ph[0], pl[0]);
+            split_bf16x8(pr + 8, ph[1], pl[1]);
+#pragma unroll
+            for (int ks2 = 0; ks2 < 2; ++ks2)
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) {
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks2][db], ph[ks2], o[db], 0, 0, 0);
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks2][db], pl[ks2], o[db], 0, 0, 0);
+                }
+            v_frags(lo, vf);
+#pragma unroll
+            for (int ks2 = 0; ks2 < 2; ++ks2)
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db)
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks2][db], ph[ks2], o[db], 0, 0, 0);
+        }
+        // slot (t + 1) % 2 was last read in step t - 1, before this step's barrier
+        if (t + 1 < nsteps) store_split((t + 1) & 1);
+        if (t + 2 < nsteps) {
+            load_raw(npg0, npg1);
+            tile_pages(kt0 + KH * (t + 3) + half, npg0, npg1);
+        }
+    }
+    if (__syncthreads_or(not_finite)) {
+        // a column that sees such a value gets the NaN its product would give
+        // (the lo half of an infinity is NaN): indicator x visibility
+#pragma clang loop unroll(disable)
+        for (int it = kt0 + half; it < kt1; it += KH) {
+            tile_pages(it, pg0, pg1);
+#pragma unroll
+            for (int ks2 = 0; ks2 < 2; ++ks2) {
+                const float* vt = (const float*)a.pool + (size_t)(ks2 ? pg1 : pg0) * a.page_elems + v_block +
+                                  (size_t)kvh * kv_tile;
+                bf16x8 vis;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int key = it * 32 - foff + 16 * ks2 + 8 * (j >> 2) + 4 * h + (j & 3);
+                    vis[j] = (__bf16)(key >= 0 && key <= jmax ? 1.0f : 0.0f);
+                }
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) {
+                    bf16x8 ind;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const float x =
+                            vt[page_order<float>(v_off(8 * (j >> 2) + 4 * h + (j & 3), 32 * db + (lane & 31)))];
+                        ind[j] = (__bf16)(__builtin_isfinite(x) ? 0.0f : 1.0f);
+                    }
+                    f32x16 seen;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) seen[i] = 0.0f;
+                    seen = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ind, vis, seen, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        if (seen[i] > 0.0f) o[db][i] = NAN;
+                }
+            }
+        }
+    }
+    prefill_finish<D, KH>(a, spl, o, m, lsum, (float*)&lds[0][0][0][0], half, wq, lane, kvh, g, grow, valid);
 }
 
 // Merge the splits of one (tile, kv head) with more than one split:
@@ -1141,37 +1387,45 @@ static zr_status launch_attn_t(zr_context* ctx, StagedMeta* st, int layer, const
                                ctx->stream, a);
         ZR_LAUNCH_CHECK(ctx);
     }
-    if constexpr (sizeof(KV) == 2) {
-        if (st->n_pblocks > 0) {
-            PrefillArgs pa;
-            pa.q = q;
-            pa.q_cols = a.q_cols;
-            pa.pool = (const uint16_t*)a.pool;
-            pa.page_elems = a.page_elems;
-            pa.stride = a.stride;
-            pa.first_offset = st->first_offset;
-            pa.kv_before = st->kv_before;
-            pa.cu_q = st->cu_q;
-            pa.blocks = st->pblocks;
-            pa.splits = st->psplits;
-            pa.n_blocks = st->n_pblocks;
-            pa.part = ctx->attn_part;
-            pa.G = a.G;
-            pa.kv_heads = a.kv_heads;
-            pa.scale_log2 = a.scale_log2;
-            pa.out_f32 = out;
-            pa.out_bf16 = out_bf16;
-            pa.out_lo_offset = a.out_lo_offset;
-            // one workgroup per (block, kv head): kv head = block index mod kv_heads, so
-            // with kv_heads dividing 8 a kv head's pages stay on the XCDs it maps to
+    if (st->n_pblocks > 0) {
+        PrefillArgs pa;
+        pa.q = q;
+        pa.q_cols = a.q_cols;
+        pa.pool = a.pool;
+        pa.page_elems = a.page_elems;
+        pa.stride = a.stride;
+        pa.first_offset = st->first_offset;
+        pa.kv_before = st->kv_before;
+        pa.cu_q = st->cu_q;
+        pa.blocks = st->pblocks;
+        pa.splits = st->psplits;
+        pa.n_blocks = st->n_pblocks;
+        pa.part = ctx->attn_part;
+        pa.G = a.G;
+        pa.kv_heads = a.kv_heads;
+        pa.scale_log2 = a.scale_log2;
+        pa.out_f32 = out;
+        pa.out_bf16 = out_bf16;
+        pa.out_lo_offset = a.out_lo_offset;
+        // one workgroup per (block, kv head): kv head = block index mod kv_heads, so
+        // with kv_heads dividing 8 a kv head's pages stay on the XCDs it maps to
+        const dim3 grid(st->n_pblocks * ctx->local_kv_heads), block(256 * st->prefill_kh);
+        if constexpr (sizeof(KV) == 2) {
             if (st->prefill_kh == 2)
-                hipLaunchKernelGGL((paged_prefill_attention_kernel<D, 4, 2>), dim3(st->n_pblocks * ctx->local_kv_heads),
-                                   dim3(512), 0, ctx->stream, pa, st->block_tables);
+                hipLaunchKernelGGL((paged_prefill_attention_kernel<D, 4, 2>), grid, block, 0, ctx->stream, pa,
+                                   st->block_tables);
             else
-                hipLaunchKernelGGL((paged_prefill_attention_kernel<D, 4, 1>), dim3(st->n_pblocks * ctx->local_kv_heads),
-                                   dim3(256), 0, ctx->stream, pa, st->block_tables);
-            ZR_LAUNCH_CHECK(ctx);
+                hipLaunchKernelGGL((paged_prefill_attention_kernel<D, 4, 1>), grid, block, 0, ctx->stream, pa,
+                                   st->block_tables);
+        } else {
+            if (st->prefill_kh == 2)
+                hipLaunchKernelGGL((paged_prefill_attention_f32_kernel<D, 2>), grid, block, 0, ctx->stream, pa,
+                                   st->block_tables);
+            else
+                hipLaunchKernelGGL((paged_prefill_attention_f32_kernel<D, 1>), grid, block, 0, ctx->stream, pa,
+                                   st->block_tables);
         }
+        ZR_LAUNCH_CHECK(ctx);
     }
     timing_mark_end(ctx, kClassAttention, ev);
     if (st->grid_merge > 0) {

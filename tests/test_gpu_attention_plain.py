@@ -30,7 +30,7 @@ def run_attention(heads, kv_heads, D, kv_dtype, cases, rng, edit=None, before=No
     Q, KV = heads * D, kv_heads * D
     geo = ModelGeometry(hidden=Q, num_heads=heads, num_kv_heads=kv_heads, num_layers=1, vocab=32, ffn=32)
     T = sum(c for _, c, _ in cases)
-    ctx = DeviceContext(geo, kv_dtype=kv_dtype, max_tokens=T, max_seqs=len(cases), max_pages_per_seq=64)
+    ctx = DeviceContext(geo, kv_dtype=kv_dtype, max_tokens=T, max_seqs=len(cases), max_pages_per_seq=200)
     ctx.create_kv_pool(sum((t + p + c + 15) // 16 + 1 for p, c, t in cases))
     if before:
         before(ctx)
