@@ -342,9 +342,8 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     st->prefill_kh = kh;
     // Prefill blocks split along their key tiles (32 keys each) when the
     // blocks alone leave CUs idle: about 512 / kh workgroups (the resident
-    // slots: 2 / kh per CU), at least 16 kh key tiles per split.  Blocks that
-    // fill the slots by themselves run unsplit (the 2108-row mixed
-    // microbatch, 64 blocks x 8 kv heads, with 4-wave workgroups: 7.82-7.88 ms
+    // slots: 2 / kh per CU).  Blocks that fill the slots by themselves run
+    // unsplit (the 2108-row mixed microbatch, 64 blocks x 8 kv heads, with 4-wave workgroups: 7.82-7.88 ms
     // per microbatch against 7.97-8.02 with 33-tile splits, whose merge takes
     // 0.19 of the 0.91 ms of attention + merge per 4 layers; running the
     // prefill kernel on a second stream beside the decode rows' attention
@@ -352,14 +351,19 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     // partials per 16-column group (16 / G rows x G heads, the decode tiles'
     // layout), one item per (group, split) after the decode items, and its
     // groups join the merge list as tiles.
-    // f32 blocks split down to 8 tiles, at most 16 splits (what the merge
-    // combines in one round trip): 64 rows on 1500, 32 / 8 heads of 128: 53 us
-    // with 8-tile splits, 62 with 16, 75 with 32; 32 rows on 6000: 71 / 64 / 84.
+    // At least 8 tiles per split and at most 16 splits, which the merge
+    // combines in one round trip (append + attention of one chunk, us, with
+    // splits of at least 32 / 16 / 8 tiles; bf16 pool, 32 q / 8 kv heads of 128:
+    // 32 rows on 2000 61 / 50 / 46, on 6000 62 / 53 / 66 (24 splits), 64 on 1500
+    // 58 / 51 / 48, 300 on 500 57 / 56 / 53; f32 pool: 64 on 1500 75 / 62 / 53).
     const long slots = 512 / kh;
-    int tps = (int)std::max<long>(f32_kv ? 8 : 16 * kh, (total_ktiles * ctx->local_kv_heads + slots - 1) / slots);
-    if (f32_kv)
-        for (const int4& b : pblk) tps = std::max(tps, ((b.w + 1) / 2 + 15) / 16);
-    if ((long)pblk.size() * ctx->local_kv_heads >= slots) tps = 1 << 30;
+    int tps = (int)std::max<long>(8, (total_ktiles * ctx->local_kv_heads + slots - 1) / slots);
+    int longest = 0;
+    for (const int4& b : pblk) longest = std::max(longest, (b.w + 1) / 2);
+    tps = std::max(tps, (longest + 15) / 16);
+    // (blocks of at most 16 tiles gain less than the merge: 512 rows, 4 kv
+    // heads of 64: 41.8 us whole, 42.6 in two splits)
+    if ((long)pblk.size() * ctx->local_kv_heads >= slots || longest <= 16) tps = 1 << 30;
     if (const char* env = getenv("ZR_ATTN_PREFILL_TILES_PER_SPLIT")) tps = std::max(1, atoi(env));
     if (G > 16) tps = 1 << 30;  // a 16-column group must hold whole rows
     int next_item = st->n_attn_items;
