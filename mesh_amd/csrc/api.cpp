@@ -742,18 +742,18 @@ zr_status zr_context_create(const zr_model_desc* desc, int device, zr_context** 
         e = hipMalloc(a.p, a.bytes);
         if (e != hipSuccess) return fail(e, "hipMalloc activations");
     }
-    // split-K workspace: max over every row count a microbatch can have (the
-    // plan changes with m, so no grid of sample sizes bounds it): 1..T rows
-    // for the layer GEMMs, 1..S for the LM head
+    // split-K workspace: max over every row count a microbatch can have: 1..T
+    // rows for the layer GEMMs, 1..S for the LM head.  The plan changes with m,
+    // past 128 rows only from one 64-row unit to the next.
     size_t ws = 0;
-    for (size_t m = 1; m <= T; ++m) {
+    for (size_t m = 1; m <= T; m = m < 128 || m == T ? m + 1 : std::min(T, m + 64)) {
         const int mm = (int)m;
         ws = std::max(ws, gemm_ws_floats(mm, (int)(Q + 2 * KV), (int)H, kEpiStore));
         ws = std::max(ws, gemm_ws_floats(mm, (int)H, (int)Q, kEpiStore));
         ws = std::max(ws, gemm_ws_floats(mm, (int)(2 * F), (int)H, kEpiSwiGLU));
         ws = std::max(ws, gemm_ws_floats(mm, (int)H, (int)F, kEpiStore));
-        if (m <= S) ws = std::max(ws, gemm_ws_floats(mm, d.vocab, (int)H, kEpiStore));
     }
+    for (size_t m = 1; m <= S; ++m) ws = std::max(ws, gemm_ws_floats((int)m, d.vocab, (int)H, kEpiStore));
     ws = std::max<size_t>(ws, 1);
     e = hipMalloc(&ctx->splitk_ws, ws * 4);
     if (e != hipSuccess) return fail(e, "hipMalloc split-K workspace");

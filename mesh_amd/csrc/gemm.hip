@@ -142,7 +142,10 @@ __device__ inline float swiglu(float g, float u) {
 // its MFMAs.)
 // Grid: 1-D, decoded so that the row blocks of one (column block, split)
 // pair are dispatched 8 apart -- on the same XCD, one after the other -- and
-// share that weight tile through its L2.
+// share that weight tile through its L2.  Pairs left over by 8 are spread
+// tile by tile: as whole pairs they gave some XCDs up to a row of tiles more
+// than the rest, often a pass over their 32 CUs  (170 tiles of
+// 2560 columns, 2108 rows, K 2048: 90 us as two passes, 50 as one).
 // SWIGLU = 1: single split; column tiles come in gate / up pairs (tile 2b is
 // gate, 2b + 1 up, WN even) and silu(g) * u is written straight to H as the
 // next GEMM's fragment-packed bf16 hi (+ lo when h_lo) operand [M, N / 2].
@@ -163,11 +166,22 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(
     typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
     __shared__ bf16x8 lds[STAGES][FSP][64];
 
-    const int b = blockIdx.x;
-    const int j = b >> 3;
-    const int rb = j % row_blocks;
-    const int g = (j / row_blocks) * 8 + (b & 7);
-    if (g >= col_blocks * splits) return;  // padding block of the XCD mapping
+    // (workgroups reach the 8 XCDs round-robin: XCD x runs the pairs x, x + 8,
+    // ...; the tiles of the last, fewer than 8, go round all XCDs)
+    const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int groups = col_blocks * splits, whole = (groups >> 3) * row_blocks;
+    int g, rb;
+    if (j < whole) {
+        g = j / row_blocks;
+        rb = j - g * row_blocks;
+        g = 8 * g + x;
+    } else {
+        const int t = (j - whole) * 8 + x;
+        g = t / row_blocks;
+        rb = t - g * row_blocks;
+        g += groups & ~7;
+        if (g >= groups) return;  // padding block
+    }
     const int cb = g / splits, split = g - cb * splits;
 
     // the wave index is uniform: readfirstlane keeps it (and every copy
@@ -550,7 +564,6 @@ zr_status launch_to_bf16_pair(zr_context* ctx, const float* x, int rows, int K, 
 // Tile configurations: wave tile WM x WN 32x32 tiles, WAVES_M x WAVES_N waves.
 struct GemmCfg {
     int wm, wn, waves_m, waves_n, stages;
-    bool small;  // many blocks per CU (weight streaming) rather than one
     int bm() const { return waves_m * wm * 32; }
     int bn() const { return waves_n * wn * 32; }
 };
@@ -564,64 +577,137 @@ static int device_cus() {
     return cus;
 }
 
-// Measured on MI355X over the decode shapes with weights streamed from HBM
-// (split activations): 32 x 128 tiles for <= 32 rows; 128-row tiles with
-// 256 columns, or 512 for wide / deep products and the LM head.
-static GemmCfg pick_cfg(int m, int n, int k, int epilogue = kEpiStore) {
-    // A vocabulary-wide head over 129-256 rows (the 256-session decode step):
-    // 256 x 256 tiles in 16-wave blocks, four waves per SIMD (128256 columns,
-    // weights streamed from HBM: 319 us against 339 us with 8-wave 256 x 256
-    // blocks).  The same blocks for the other decode products measured no
-    // faster (gate / up) or slower; 64-row tiles, two blocks per CU, are
-    // faster only while the weights sit in the last-level cache.
-    if (m > 128 && m <= 256 && epilogue == kEpiStore && n >= 65536) return {2, 2, 4, 4, 3, false};
-    // SwiGLU fused into the GEMM (one split, gate / up tile pairs in a wave) once
-    // 128-row tiles fill the CUs; small row counts reduce split-K slabs instead.
-    // 128 x 512 tiles once they alone fill two passes over the CUs (prefill-sized
-    // row counts: gate/up at 2108 rows 838-850 us against 910-1117 with 128 x 256).
-    if (epilogue == kEpiSwiGLU && m > 64) {
-        const int wide_tiles = ((m + 127) / 128) * ((n + 511) / 512);
-        if (wide_tiles >= 2 * device_cus()) return {2, 4, 2, 4, 3, false};
-        // 65-128 rows: 64 x 256 tiles (two row blocks share each weight tile)
-        // fill twice the CUs of one 128-row block (decode steps at 96 / 128
-        // sessions -4.7 / -4.2 %); at 256 rows they are slower (GEMMs 7.5
-        // against 6.8 ms per step)
-        if (m <= 128) return {2, 2, 1, 4, 3, false};
-        // 129-256 rows: the same 128 x 256 tiles in 16-wave blocks (32 x 64
-        // wave tiles, four waves per SIMD to cover the copies' latency):
-        // GEMM class 7.33-7.36 against 7.47-7.50 ms per 256-session step with
-        // 8 waves.  The store products measured slower in 16-wave blocks.
-        if (m <= 256) return {1, 2, 4, 4, 3, false};
-        return {2, 2, 2, 4, 3, false};
-    }
-    // <= 32 rows: a 4-deep ring and one pass of splits over the CUs (TinyLlama
-    // shapes at 32 rows, back to back with weights from HBM: QKV 4.84 us
-    // against 5.27 with 3 stages and three blocks per CU, gate/up 15.6 against
-    // 17.1 (2 slabs instead of 8 for the SwiGLU reduce), down 6.96 against
-    // 7.48, LM head 26.8 unsplit against 28.2 + its reduce; O unchanged)
-    if (m <= 32) return {1, 1, 1, 4, 4, false};
-    // 33-64 rows the same way on 64-row tiles (the tensor-parallel shard step
-    // at 64 sessions: 12.6k -> 13.4k tokens/s against ~3 blocks per CU and 3
-    // stages, whose 16 slabs each consumer read back)
-    if (m <= 64) return {2, 1, 1, 4, 4, false};
-    // and the 65-128-row store products (QKV, O, down) on two or more 64-row
-    // tiles: fewer split-K slabs for their consumers (decode steps at 96 / 128
-    // sessions 10.5 -> 10.2 / 12.4 -> 11.3 ms; at 128 sessions the attention,
-    // with RoPE inside, sums q from 2 QKV slabs instead of 10).  At 256 rows
-    // the same plan costs the GEMMs what it saves their consumers.
-    if (m <= 128 && epilogue == kEpiStore && n < 65536) return {2, 1, 1, 4, 4, false};
-    // vocabulary-wide heads: 256-row tiles read each weight tile once
-    if (n >= 65536) return m > 128 ? GemmCfg{2, 4, 4, 2, 3, false} : GemmCfg{2, 4, 2, 4, 3, false};
-    if (n >= 16384) return {2, 4, 2, 4, 3, false};
-    return {2, 2, 2, 4, 3, false};
-}
-
 static bool swiglu_fused(int m, int epilogue) { return epilogue == kEpiSwiGLU && m > 64; }
 
 // <= 64 rows of gate / up: SwiGLU in one launch with K split over the waves of
 // a workgroup (gemm_swiglu_ksplit_kernel; two 32-row tiles above 32 rows)
 static bool swiglu_ksplit(int m, int n, int k, int epilogue) {
     return epilogue == kEpiSwiGLU && m <= 64 && n % 64 == 0 && ((k + 31) / 32) % 4 == 0;
+}
+
+struct GemmChoice {
+    GemmCfg cfg;
+    int splits;
+};
+
+// Split K as far as the grid fits one pass over the CUs, >= 4 k-steps per
+// split, at most 16 splits.  More tiles than one pass: up to 4 splits when they
+// fill the last pass better, in passes of unsplit blocks plus, per extra split,
+// one more f32 slab written and read back (8 M N bytes at ~5 TB/s) against one
+// pass of the hi + lo MFMA work (4 BM BN K per CU at ~1.2 PFLOP/s).
+static GemmChoice one_pass(const GemmCfg& c, int m, int n, int k) {
+    const int tiles = ((m + c.bm() - 1) / c.bm()) * ((n + c.bn() - 1) / c.bn());
+    const int KT = (k + 31) / 32, cus = device_cus();
+    if (tiles <= cus) return {c, std::max(1, std::min(std::min(16, cus / tiles), KT / 4))};
+    const double slab = 480.0 * tiles / ((double)k * cus);
+    GemmChoice best{c, 1};
+    double least = 1e30;
+    for (int s = 1; s <= 4 && s <= std::max(1, KT / 4); ++s) {
+        const double cost = (double)(((size_t)tiles * s + cus - 1) / cus) / s + slab * (s - 1);
+        if (cost < least - 1e-9) {
+            least = cost;
+            best.splits = s;
+        }
+    }
+    return best;
+}
+
+// Tiles of products over many rows, priced by how they fill the CUs.  A block
+// of a config takes `step` us per k-step of 32 (plus four of prologue and
+// epilogue) in a full pass over its slots; a last pass over a share f of them
+// takes alone + (1 - alone) f of that, less than a whole one because the chip
+// clocks higher then (it runs these products at its power limit: full passes
+// reach 1.34-1.44 PFLOP/s of MFMA work whatever the tile).  Fitted to cold
+// weights, hi + lo operands, 256-3000 rows, 2048-28672 columns, K 2048-14336;
+// within 5 % of most of them.  With two blocks per CU, up to half of the slots
+// run one to a CU.
+struct TileCost {
+    GemmCfg cfg;
+    int per_cu;
+    float step, alone;
+};
+static const TileCost kTileCosts[] = {
+    {{2, 2, 2, 4, 3}, 1, 0.80f, 0.70f},  // 128 x 256
+    {{2, 2, 3, 4, 3}, 1, 1.10f, 0.60f},  // 192 x 256, 12 waves
+    {{2, 2, 4, 4, 3}, 1, 1.47f, 0.50f},  // 256 x 256, 16 waves
+    {{2, 2, 1, 4, 3}, 2, 0.90f, 0.70f},  // 64 x 256, two blocks per CU
+};
+
+static GemmChoice cheapest(int m, int n, int k, bool may_split) {
+    // priced at whole 64-row units, so that a plan (and its workspace) changes
+    // at their ends only
+    const int rows = (m + 63) / 64 * 64, KT = (k + 31) / 32, cus = device_cus();
+    GemmChoice best{kTileCosts[0].cfg, 1};
+    float least = 1e30f;
+    for (const TileCost& t : kTileCosts) {
+        const int tiles = ((rows + t.cfg.bm() - 1) / t.cfg.bm()) * ((n + t.cfg.bn() - 1) / t.cfg.bn());
+        const int slots = t.per_cu * cus;
+        for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
+            if (s > 1 && KT / s < 4) break;
+            if (s > 4 && tiles * s > 2 * cus) break;  // (bounds the workspace)
+            const int blocks = tiles * s, full = blocks / slots;
+            const float f = (float)(blocks - full * slots) / slots;
+            float passes = (float)full;
+            if (f > 0.0f)
+                passes += t.per_cu == 2 && f <= 0.5f ? 0.45f + 0.15f * f : t.alone + (1.0f - t.alone) * f;
+            // each split past the first: one more f32 slab written and read at ~5 TB/s
+            const float us = passes * t.step * ((KT + s - 1) / s + 4) + 8e-6f / 5 * rows * (float)n * (s - 1);
+            if (us < least) {
+                least = us;
+                best = {t.cfg, s};
+            }
+        }
+    }
+    return best;
+}
+
+// The tile and K split of a product (measured with weights streamed from HBM
+// and split activations; the decode steps are those of TinyLlama and Llama-3
+// shapes).
+static GemmChoice choose_tiles(int m, int n, int k, int epilogue) {
+    const bool store = epilogue == kEpiStore;
+    // A vocabulary-wide head over 129-256 rows (the 256-session decode step):
+    // 256 x 256 tiles in 16-wave blocks, four waves per SIMD (128256 columns:
+    // 319 us against 339 us with 8-wave 256 x 256 blocks).
+    if (m > 128 && m <= 256 && store && n >= 65536) return one_pass({2, 2, 4, 4, 3}, m, n, k);
+    if (swiglu_fused(m, epilogue)) {
+        // 65-128 rows: 64 x 256 tiles (two row blocks share each weight tile)
+        // fill twice the CUs of one 128-row block (decode steps at 96 / 128
+        // sessions -4.7 / -4.2 %)
+        if (m <= 128) return {{2, 2, 1, 4, 3}, 1};
+        const GemmChoice c = cheapest(m, n, k, false);
+        // 129-256 rows: 128 x 256 tiles in 16-wave blocks (32 x 64 wave tiles,
+        // four waves per SIMD to cover the copies' latency): GEMM class
+        // 7.33-7.36 against 7.47-7.50 ms per 256-session step with 8 waves.
+        // The store products measured slower in 16-wave blocks.
+        if (m <= 256 && c.cfg.bm() == 128) return {{1, 2, 4, 4, 3}, 1};
+        return c;
+    }
+    // <= 32 rows: a 4-deep ring and one pass of splits over the CUs (TinyLlama
+    // shapes at 32 rows, back to back with weights from HBM: QKV 4.84 us
+    // against 5.27 with 3 stages and three blocks per CU, gate/up 15.6 against
+    // 17.1 (2 slabs instead of 8 for the SwiGLU reduce), down 6.96 against
+    // 7.48, LM head 26.8 unsplit against 28.2 + its reduce; O unchanged)
+    if (m <= 32) return one_pass({1, 1, 1, 4, 4}, m, n, k);
+    // 33-64 rows the same way on 64-row tiles (the tensor-parallel shard step
+    // at 64 sessions: 12.6k -> 13.4k tokens/s against ~3 blocks per CU and 3
+    // stages, whose 16 slabs each consumer read back)
+    if (m <= 64) return one_pass({2, 1, 1, 4, 4}, m, n, k);
+    // and the 65-128-row store products (QKV, O, down) on two or more 64-row
+    // tiles: fewer split-K slabs for their consumers (decode steps at 96 / 128
+    // sessions 10.5 -> 10.2 / 12.4 -> 11.3 ms; at 128 sessions the attention,
+    // with RoPE inside, sums q from 2 QKV slabs instead of 10).  At 256 rows
+    // the same plan costs the GEMMs what it saves their consumers.
+    if (m <= 128 && store && n < 65536) return one_pass({2, 1, 1, 4, 4}, m, n, k);
+    // vocabulary-wide heads: 256-row tiles read each weight tile once
+    if (n >= 65536) return one_pass(m > 128 ? GemmCfg{2, 4, 4, 2, 3} : GemmCfg{2, 4, 2, 4, 3}, m, n, k);
+    if (m <= 256) return one_pass(n >= 16384 ? GemmCfg{2, 4, 2, 4, 3} : GemmCfg{2, 2, 2, 4, 3}, m, n, k);
+    // More rows (us per product, the rules before -- 128 x 256 tiles, up to 4
+    // splits past one pass -- against these): Llama-3 at 2108 rows QKV 198 /
+    // 186, O 143 / 135 and no slabs, down 436 / 424 (no slabs), at 997 gate/up
+    // 401 / 374, at 520 288 / 232; TinyLlama at 997 gate/up 104 / 89, at 2108
+    // QKV 90 / 50, down 118 / 93.
+    return cheapest(m, n, k, true);
 }
 
 GemmPlan gemm_plan(int m, int n, int k, int epilogue) {
@@ -634,36 +720,18 @@ GemmPlan gemm_plan(int m, int n, int k, int epilogue) {
         p.kt_per_split = p.KT;
         return p;  // one launch, no workspace
     }
-    const GemmCfg c = pick_cfg(m, n, k, epilogue);
+    const GemmChoice ch = choose_tiles(m, n, k, epilogue);
+    const GemmCfg& c = ch.cfg;
+    p.wm = c.wm;
+    p.wn = c.wn;
+    p.waves_m = c.waves_m;
+    p.waves_n = c.waves_n;
+    p.stages = c.stages;
     p.KT = (k + 31) / 32;
     p.NT = (n + 31) / 32;
     p.row_blocks = (m + c.bm() - 1) / c.bm();
     p.col_blocks = (p.NT + c.bn() / 32 - 1) / (c.bn() / 32);
-    // split K as far as the grid fits one pass over the CUs (one resident
-    // block per CU for the large tiles, about three for the small
-    // weight-streaming tiles), >= 4 k-steps per split, at most 16 splits
-    const int tiles = p.col_blocks * p.row_blocks;
-    const int budget = c.small ? 3 * device_cus() : device_cus();
-    int splits = swiglu_fused(m, epilogue) ? 1 : std::max(1, std::min(std::min(16, budget / tiles), p.KT / 4));
-    if (!swiglu_fused(m, epilogue) && !c.small && tiles > budget) {
-        // More tiles than one pass: up to 4 splits when they fill the last
-        // pass better.  Cost in passes of unsplit blocks: ceil(tiles S / CUs) / S,
-        // plus per extra split one more f32 slab written and read back
-        // (8 M N bytes at ~5 TB/s) against one pass of the hi + lo MFMA work
-        // (4 BM BN K per CU at ~1.2 PFLOP/s): 480 tiles / (K CUs).  At 2108 rows
-        // this picks S = 3 for O (K 4096) and 4 for down (K 14336): -20 to -30 %
-        // per GEMM; QKV's slabs cost more than its tail (S = 1).
-        const double slab = 480.0 * tiles / ((double)k * budget);
-        double best = 1e30;
-        for (int s = 1; s <= 4 && s <= std::max(1, p.KT / 4); ++s) {
-            const double cost = (double)(((size_t)tiles * s + budget - 1) / budget) / s + slab * (s - 1);
-            if (cost < best - 1e-9) {
-                best = cost;
-                splits = s;
-            }
-        }
-    }
-    p.kt_per_split = (p.KT + splits - 1) / splits;
+    p.kt_per_split = (p.KT + ch.splits - 1) / ch.splits;
     p.splits = (p.KT + p.kt_per_split - 1) / p.kt_per_split;
     p.direct = p.splits == 1 && (epilogue == kEpiStore || swiglu_fused(m, epilogue));
     p.ws_floats = p.direct ? 0 : (size_t)p.splits * m * n;
@@ -673,8 +741,7 @@ GemmPlan gemm_plan(int m, int n, int k, int epilogue) {
 template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, int HL, int SWIGLU = 0>
 static void gemm_launch(const GemmPlan& p, hipStream_t stream, const uint16_t* a, int m, int k, const uint16_t* w,
                         float* c, int n, size_t split_stride, uint16_t* h = nullptr, int h_lo = 0) {
-    const int groups = p.col_blocks * p.splits;
-    const unsigned blocks = 8u * (unsigned)p.row_blocks * (unsigned)((groups + 7) / 8);
+    const unsigned blocks = ((unsigned)p.row_blocks * (unsigned)p.col_blocks * (unsigned)p.splits + 7u) / 8u * 8u;
     hipLaunchKernelGGL((gemm_kernel<WM, WN, WAVES_M, WAVES_N, HL, STAGES, SWIGLU>), dim3(blocks),
                        dim3(WAVES_M * WAVES_N * 64), 0, stream, a, m, k, (const bf16x8*)w, p.KT, p.NT, c, n,
                        p.kt_per_split, p.splits, p.row_blocks, p.col_blocks, split_stride, h, h_lo);
@@ -717,7 +784,6 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
         return ZR_OK;
     }
     const GemmPlan p = gemm_plan(m, n, k, epilogue);
-    const GemmCfg cfg = pick_cfg(m, n, k, epilogue);
     if (swiglu_fused(m, epilogue) && (!c_bf16 || c_f32 || n % 64 != 0))
         return set_err(ctx, ZR_E_INVARIANT, "fused SwiGLU writes the bf16 operand only (N=%d)", n);
     const bool fused = swiglu_fused(m, epilogue);
@@ -730,22 +796,23 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
     timing_mark_begin(ctx, kClassGemm, &ev);
     bool launched = false;
 #define ZR_GEMM_FUSED_CASE(WMV, WNV, WAM, WAN, ST)                                                     \
-    if (fused && !launched && cfg.wm == WMV && cfg.wn == WNV && cfg.waves_m == WAM &&                  \
-        cfg.waves_n == WAN && cfg.stages == ST) {                                                      \
+    if (fused && !launched && p.wm == WMV && p.wn == WNV && p.waves_m == WAM && p.waves_n == WAN &&    \
+        p.stages == ST) {                                                                              \
         if (split_act)                                                                                 \
             gemm_launch<WMV, WNV, WAM, WAN, ST, 2, 1>(p, ctx->stream, a, m, k, w_packed, nullptr, n, 0, c_bf16, 1); \
         else                                                                                           \
             gemm_launch<WMV, WNV, WAM, WAN, ST, 1, 1>(p, ctx->stream, a, m, k, w_packed, nullptr, n, 0, c_bf16, 0); \
         launched = true;                                                                               \
     }
-    ZR_GEMM_FUSED_CASE(2, 4, 2, 4, 3)
     ZR_GEMM_FUSED_CASE(2, 2, 2, 4, 3)
     ZR_GEMM_FUSED_CASE(2, 2, 1, 4, 3)
     ZR_GEMM_FUSED_CASE(1, 2, 4, 4, 3)
+    ZR_GEMM_FUSED_CASE(2, 2, 3, 4, 3)
+    ZR_GEMM_FUSED_CASE(2, 2, 4, 4, 3)
 #undef ZR_GEMM_FUSED_CASE
 #define ZR_GEMM_CASE(WMV, WNV, WAM, WAN, ST)                                                           \
-    if (!fused && !launched && cfg.wm == WMV && cfg.wn == WNV && cfg.waves_m == WAM &&                 \
-        cfg.waves_n == WAN && cfg.stages == ST) {                                                      \
+    if (!fused && !launched && p.wm == WMV && p.wn == WNV && p.waves_m == WAM && p.waves_n == WAN &&   \
+        p.stages == ST) {                                                                              \
         if (split_act)                                                                                 \
             gemm_launch<WMV, WNV, WAM, WAN, ST, 2>(p, ctx->stream, a, m, k, w_packed, dst, n, split_stride); \
         else                                                                                           \
@@ -753,8 +820,9 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
         launched = true;                                                                               \
     }
     ZR_GEMM_CASE(1, 1, 1, 4, 4)
-    ZR_GEMM_CASE(2, 1, 1, 4, 3)
     ZR_GEMM_CASE(2, 1, 1, 4, 4)
+    ZR_GEMM_CASE(2, 2, 1, 4, 3)
+    ZR_GEMM_CASE(2, 2, 3, 4, 3)
     ZR_GEMM_CASE(2, 2, 4, 4, 3)
     ZR_GEMM_CASE(2, 4, 4, 2, 3)
     ZR_GEMM_CASE(2, 4, 2, 4, 3)
