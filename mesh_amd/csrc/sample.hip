@@ -29,14 +29,15 @@
 //   full distribution: one pass of weight sums over 16 contiguous ranges
 //     (one per wave), then the range holding the crossing.
 //   nucleus: the (p descending, index ascending) order is never built.  One
-//     pass histograms e by exponent and two mantissa bits (weight sums), which
-//     fixes the bucket of the top_p crossing and the range of buckets the
+//     pass histograms e by exponent and four mantissa bits (weight sums; the
+//     elements below 2^-14, most of a row, only add to one sum, and a second
+//     pass places them if the top_p crossing lies among them), which fixes the bucket of the top_p crossing and the range of buckets the
 //     sampled crossing can fall in; when those buckets hold at most 8192
 //     elements (bounded by weight sum / smallest weight), one pass collects
 //     them into LDS, they are sorted by (e, -index) (by rank up to 1024 of
 //     them, a bitonic network beyond) and both crossings are read off the
 //     sorted run.  Otherwise each crossing is
-//     refined on its own: further passes over the next 11 and 10 bits,
+//     refined on its own: further passes over the next 10 and 9 bits,
 //     collection of the bucket, and, for a run of more than 8192 equal
 //     probabilities, rank in index order by per-tile counts.
 #include "zr_internal.h"
@@ -55,8 +56,16 @@ constexpr int kCap = 8192;                     // candidates resolved in LDS
 constexpr int kMaxCols = 1 << 20;              // weight sums stay below 2^57
 constexpr uint32_t kMinKey = 90u << 23;        // e < 2^-37 weighs 0
 constexpr uint32_t kOneKey = 127u << 23;       // e == 1
-constexpr int kL1Base = (int)(kMinKey >> 21);  // first level: bits 21..31, offset
-constexpr int kL1Buckets = 256;
+// First level: bits 19..31, offset.  Two mantissa bits instead of four put
+// thousands of elements of a flat row into the crossing's bucket, which are
+// then sorted or refined (256 rows x 128256 N(0, 9), the call: T 1.3, top_p
+// 0.95 258 us against 186, T 0.85, top_p 0.9 119 against 104, T 0.7 101 against
+// 98; one row of 32000: 76 against 50, T 0.7 41 against 42; five bits gain more
+// on flat rows -- 152 us -- and cost the others 2 us).
+constexpr int kL1Shift = 19;
+constexpr int kL1Base = (int)(kMinKey >> kL1Shift);
+constexpr int kL1Buckets = (int)(kOneKey >> kL1Shift) - kL1Base + 1;  // 593
+constexpr uint32_t kSplitKey = 113u << 23;     // 2^-14
 constexpr float kLog2E = 1.44269504088896341f;
 
 struct SampleRowArgs {
@@ -80,6 +89,20 @@ __device__ inline uint64_t fix_weight(uint32_t b) {
     return eb > 127u ? 0 : w;
 }
 
+// The same for e < 2^-5: x = e 2^36 below 2^31 is exact, and so is its distance
+// to the integer below it.  Not a number: 0.
+__device__ inline uint32_t fix_weight_small(float e) {
+    const float x = fmaxf(e * 0x1p36f, 0.0f);
+    const uint32_t u = (uint32_t)x;
+    return u + (x - (float)u >= 0.5f ? 1u : 0u);
+}
+
+// fix_weight of e, the 64-bit shift only where a lane of the wave needs it
+__device__ inline uint64_t fix_weight_of(float e) {
+    if (__any(e >= 0x1p-5f)) return fix_weight(__float_as_uint(e));
+    return fix_weight_small(e);
+}
+
 // ceil(a * b / 2^q) for a * b < 2^120.
 __device__ inline uint64_t ceil_mul_shr(uint64_t a, uint64_t b, int q) {
     const unsigned __int128 p = (unsigned __int128)a * b;
@@ -87,8 +110,8 @@ __device__ inline uint64_t ceil_mul_shr(uint64_t a, uint64_t b, int q) {
     return (uint64_t)((p + (((unsigned __int128)1 << q) - 1)) >> q);
 }
 
-__device__ inline int l1_bucket(uint32_t key) { return (int)(key >> 21) - kL1Base; }
-__device__ inline uint64_t l1_min_weight(int b) { return fix_weight((uint32_t)(b + kL1Base) << 21); }
+__device__ inline int l1_bucket(uint32_t key) { return (int)(key >> kL1Shift) - kL1Base; }
+__device__ inline uint64_t l1_min_weight(int b) { return fix_weight((uint32_t)(b + kL1Base) << kL1Shift); }
 
 struct Row {
     const float* x;
@@ -214,6 +237,7 @@ struct Shared {
     uint64_t off[kL1Buckets];    // running-weight offset of collected buckets
     uint64_t cand[kCap];         // (e bits << 32) | (~column), sorted descending
     uint64_t wtot[kWaves];
+    uint64_t part[16];           // weight below the split, by thread index
     float fm[kWaves];
     int fi[kWaves];
     int ncand, bucket, found, first;
@@ -478,12 +502,12 @@ __device__ __attribute__((always_inline)) inline int refine_cross(const Row& R, 
     const int tid = threadIdx.x;
     hist_cross(S.hist1, kL1Buckets, true, target, 0, S);
     if (S.bucket < 0) return -1;
-    uint32_t mask = 0xFFE00000u, value = (uint32_t)(S.bucket + kL1Base) << 21;
+    uint32_t mask = ~((1u << kL1Shift) - 1), value = (uint32_t)(S.bucket + kL1Base) << kL1Shift;
     uint64_t acc = S.acc, bsum = S.bsum;
     int level = 1;
     // elements in a bucket <= its weight / the weight of its smallest key
     while (bsum / fix_weight(value) > (uint64_t)kCap && level < 3) {
-        const int sh = level == 1 ? 10 : 0, nb = level == 1 ? 2048 : 1024;
+        const int sh = level == 1 ? 9 : 0, nb = level == 1 ? 1 << (kL1Shift - 9) : 512;
         for (int b = tid; b < nb; b += kThreads) S.hist[b] = 0;
         __syncthreads();
         sweep(R, [&](int, float v, int) {
@@ -595,7 +619,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
         // wave sums a contiguous range, the crossing range is scanned
         const int span = (((cols + kWaves - 1) / kWaves) + 3) & ~3;
         uint64_t sum = 0;
-        sweep_wave_range(R, span, [&](int, float v) { sum += fix_weight(R.key(v)); });
+        sweep_wave_range(R, span, [&](int, float v) { sum += fix_weight_of(__uint_as_float(R.key(v))); });
 #pragma unroll
         for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o, 64);
         if (lane == 0) S.hist[wave] = sum;
@@ -616,19 +640,42 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     }
     // nucleus: the first-level histogram and each bucket's preceding weight
     for (int b = tid; b < kL1Buckets; b += kThreads) S.hist1[b] = 0;
+    if (tid < 16) S.part[tid] = 0;
     __syncthreads();
+    uint64_t rest = 0;
     sweep(R, [&](int, float v, int) {
         const uint32_t key = R.key(v);
-        const uint64_t w = fix_weight(key);
-        if (w) atomicAdd((unsigned long long*)&S.hist1[l1_bucket(key)], (unsigned long long)w);
+        if (key >= kSplitKey && key <= kOneKey)
+            atomicAdd((unsigned long long*)&S.hist1[l1_bucket(key)], (unsigned long long)fix_weight(key));
+        else
+            rest += fix_weight_small(__uint_as_float(key));
     });
-    __syncthreads();
+    if (rest) atomicAdd((unsigned long long*)&S.part[tid & 15], (unsigned long long)rest);
+    static_assert(kL1Buckets <= kThreads, "a bucket per thread");
     uint64_t total;
-    {
+    auto weights_above = [&]() {
         const int b = kL1Buckets - 1 - tid;  // descending
-        const uint64_t mine = b >= 0 ? S.hist1[b] : 0;
-        const uint64_t ex = block_exscan(mine, S, &total);
+        const uint64_t ex = block_exscan(b >= 0 ? S.hist1[b] : 0, S, &total);
         if (b >= 0) S.pre1[b] = ex;
+    };
+    __syncthreads();
+    weights_above();
+    uint64_t below = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) below += S.part[i];
+    // the last kept element: first with cum >= P (none when P > W: all kept)
+    const uint64_t P = ceil_mul_shr(a.tp_m, total + below, a.tp_q);
+    if (below && P > total) {
+        // the last kept element lies below the split: place the rest too
+        sweep(R, [&](int, float v, int) {
+            const uint32_t key = R.key(v);
+            const uint32_t w = key < kSplitKey ? fix_weight_small(__uint_as_float(key)) : 0u;
+            if (w) atomicAdd((unsigned long long*)&S.hist1[l1_bucket(key)], (unsigned long long)w);
+        });
+        __syncthreads();
+        weights_above();
+    } else {
+        total += below;
     }
     if (tid == 0) S.bucket = -1;
     __syncthreads();
@@ -636,10 +683,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
         if (tid == 0) out[r] = 0;
         return;
     }
-    // the last kept element: first with cum >= P (none when P > W: all kept);
     // the first-level buckets holding running weight P, then the range the
     // sampled target ceil(k * denom / 2^24) can reach, denom within bucket b1
-    const uint64_t P = ceil_mul_shr(a.tp_m, total, a.tp_q);
     auto holds = [&](int b, uint64_t t) { return S.hist1[b] && S.pre1[b] < t && t <= S.pre1[b] + S.hist1[b]; };
     if (tid < kL1Buckets && P <= total && holds(tid, P)) S.bucket = tid;
     __syncthreads();
@@ -670,13 +715,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     if (bl >= 0 && bh >= 0 && bound <= (uint64_t)kCap) {
         // both crossings from one collected, sorted run
         // the set is b1 and bl..bh (b1 <= bl): one key range when adjacent
-        const uint32_t lo_b1 = (uint32_t)(b1 + kL1Base) << 21, lo_bl = (uint32_t)(bl + kL1Base) << 21;
-        const uint32_t hi_bh = ((uint32_t)(bh + kL1Base + 1) << 21) - 1;
+        const uint32_t lo_b1 = (uint32_t)(b1 + kL1Base) << kL1Shift, lo_bl = (uint32_t)(bl + kL1Base) << kL1Shift;
+        const uint32_t hi_bh = ((uint32_t)(bh + kL1Base + 1) << kL1Shift) - 1;
         int n;
         if (b1 < 0 || b1 >= bl - 1)
             n = collect_sorted(R, b1 < 0 ? lo_bl : (b1 < bl ? lo_b1 : lo_bl), hi_bh, 1u, 0u, S);
         else
-            n = collect_sorted(R, lo_b1, lo_b1 + (1u << 21) - 1, lo_bl, hi_bh, S);
+            n = collect_sorted(R, lo_b1, lo_b1 + (1u << kL1Shift) - 1, lo_bl, hi_bh, S);
         {
             // running-weight offset of each collected bucket: its preceding
             // weight less the collected weight of the buckets above it
