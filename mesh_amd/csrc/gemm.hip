@@ -479,6 +479,144 @@ __global__ __launch_bounds__(256) void gemm_swiglu_ksplit_kernel(const uint16_t*
         }
 }
 
+// At most kFewRows rows (one session's step, a few of them): the product is the
+// stream of its weights, and the ring above copies a padded 32-row A tile, as
+// many bytes as the weights themselves, beside them.  Here a workgroup of NW
+// waves owns 16 columns (SWIGLU: 16 of H, a gate and an up tile), and the waves
+// take consecutive runs of its k-steps.  Weights go straight to registers as
+// v_mfma_f32_16x16x32_bf16 fragments: lane l = 16 q + i holds k 8 q + j of
+// column i, one 16-byte run of the packed 32x32x16 fragment 2 kt + q / 2 (four
+// 256-byte runs per wave load).  Of A only the MR rows (M rounded up to a power
+// of two) are read, 16-byte runs packed 64 to a load, and pass through a
+// per-wave LDS block to their fragments (as masked fragment loads, two per
+// k-step beside one of weights, the address unit held the stream back).  The
+// fragments' rows past MR repeat the others: their products are not stored.
+// Rows past M and steps past the wave's run are loads past the buffer's end:
+// zeros, and no memory traffic.  Two sets of U steps alternate, the next one in
+// flight under the other's products; the waves' sums meet in LDS and are added
+// in wave order.
+// One session's TinyLlama step (517 tokens, us per launch, before / after):
+// gate/up 14.1 / 11.9, LM head 27.3 / 23.6 (5.5 TB/s), QKV 5.2 / 5.0 and O, down
+// 5.6 / 5.3, with 1-2 slabs instead of 11-16, which take the norms from 4.3 to
+// 3.6; the step's kernels 1190 / 1080.  What is left is launch ramp: 8-46 MB at
+// the rate of the LM head would take 1.5-8.4.
+// Waves and steps per set (NW, U) tried: (4, 4), (8, 2), (8, 4), (4, 8); with
+// 9-16 rows (and 16 in masked fragment loads) the tiles are faster (Llama-3, 16
+// sessions 621 / 656 us per step of 4 layers).
+constexpr int kFewRows = 8;
+constexpr int kWeightCache = 2;  // nontemporal: read once per product
+template <int MR, int NW, int U, int HL, int SWIGLU>
+__global__ __launch_bounds__(NW * 64) void gemm_few_rows_kernel(const uint16_t* __restrict__ A, int M,
+                                                                const uint16_t* __restrict__ Wp, int KT, int NT,
+                                                                float* __restrict__ C, int N, int kt_per_split,
+                                                                int splits, size_t split_stride,
+                                                                uint16_t* __restrict__ H) {
+    constexpr int TW = SWIGLU ? 2 : 1;
+    constexpr int NA = (U * HL * 4 * MR + 63) / 64;  // loads of A runs per set
+    typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
+    __shared__ f32x4 red[NW][TW][64];
+    __shared__ u32x4 rows[NW][NA * 64];  // [step u][hi, lo][q][row]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int col16 = blockIdx.x / splits, split = blockIdx.x - col16 * splits;
+    const int q = lane >> 4, i16 = lane & 15;
+    const unsigned plane_bytes = (unsigned)KT << 11;  // one 32-row or 32-column tile: 2 KT fragments of 1 KiB
+    const __amdgpu_buffer_rsrc_t rsrc_a =
+        __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(plane_bytes * HL), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_w =
+        __builtin_amdgcn_make_buffer_rsrc((void*)Wp, 0, (int)(plane_bytes * (unsigned)NT), 0x00020000);
+    constexpr unsigned kPast = 0x80000000u;  // beyond either buffer (both below 2 GiB)
+    const unsigned tile0 = SWIGLU ? (unsigned)(col16 >> 1) * 2 : (unsigned)(col16 >> 1);
+    const unsigned w0 = tile0 * plane_bytes + (unsigned)(q >> 1) * 1024 + (unsigned)(q & 1) * 512 +
+                        (unsigned)(col16 & 1) * 256 + i16 * 16;
+    // the lane's run of A load v: byte offset at step 0 and its step within the set (U: none)
+    unsigned a0[NA];
+    int au[NA];
+#pragma unroll
+    for (int v = 0; v < NA; ++v) {
+        const int idx = v * 64 + lane, row = idx & (MR - 1), r = idx / MR, aq = r & 3, h = (r >> 2) % HL;
+        au[v] = (r >> 2) / HL;
+        a0[v] = (unsigned)h * plane_bytes + ((unsigned)au[v] << 11) + (unsigned)(aq >> 1) * 1024 +
+                (unsigned)(aq & 1) * 512 + row * 16;
+        if (row >= M || au[v] >= U) au[v] = 1 << 28;
+    }
+    // this wave's steps of the split's
+    const int kb = split * kt_per_split, n = min(KT, kb + kt_per_split) - kb;
+    const int s0 = kb + (int)((long)wave * n / NW), s1 = kb + (int)((long)(wave + 1) * n / NW);
+
+    u32x4 wr[2][U][TW], ar[2][NA];
+    auto load = [&](int set, int s) {
+#pragma unroll
+        for (int v = 0; v < NA; ++v)
+            ar[set][v] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc_a, (int)(s + au[v] < s1 ? a0[v] + ((unsigned)s << 11) : kPast), 0, 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int t = 0; t < TW; ++t)
+                wr[set][u][t] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rsrc_w, (int)(s + u < s1 ? w0 + t * plane_bytes + ((unsigned)(s + u) << 11) : kPast), 0,
+                    kWeightCache);
+    };
+    f32x4 acc[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](int set) {
+        // (one wave's LDS operations run in order; the fences keep the compiler's order the same)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int v = 0; v < NA; ++v) rows[wave][v * 64 + lane] = ar[set][v];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < HL; ++h) {
+                const bf16x8 fa =
+                    __builtin_bit_cast(bf16x8, rows[wave][((u * HL + h) * 4 + q) * MR + (i16 & (MR - 1))]);
+#pragma unroll
+                for (int t = 0; t < TW; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, __builtin_bit_cast(bf16x8, wr[set][u][t]),
+                                                                     acc[t], 0, 0, 0);
+            }
+    };
+    load(0, s0);
+    for (int s = s0; s < s1; s += 2 * U) {
+        load(1, s + U);
+        __builtin_amdgcn_sched_barrier(0);
+        products(0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(0, s + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        products(1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < TW; ++t) red[wave][t][lane] = acc[t];
+    __syncthreads();
+    // thread (m, column): element m % 4 of lane 16 (m / 4) + column
+    const int m = tid >> 4, c = tid & 15;
+    if (m >= M) return;  // (M <= 8 rows, at least 256 threads)
+    float v[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+        v[t] = red[0][t][16 * (m >> 2) + c][m & 3];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v[t] += red[w][t][16 * (m >> 2) + c][m & 3];
+    }
+    const int j = col16 * 16 + c;
+    if constexpr (SWIGLU) {
+        const int F = N / 2;
+        uint16_t hi, lo;
+        split_bf16(swiglu(v[0], v[TW - 1]), hi, lo);
+        const size_t o = a_pack_index(m, j, F);
+        H[o] = hi;
+        if (HL == 2) H[a_plane(M, F) + o] = lo;
+    } else if (j < N) {
+        C[(size_t)split * split_stride + (size_t)m * N + j] = v[0];
+    }
+}
+
 // Sum of split-K slabs [S][M][N] with the epilogue.
 // kEpiStore:  out_f32[m][n] = sum
 // kEpiSwiGLU: N = 2F interleaved per 32 columns; h = silu(g) * u written as
@@ -584,6 +722,11 @@ static bool swiglu_fused(int m, int epilogue) { return epilogue == kEpiSwiGLU &&
 static bool swiglu_ksplit(int m, int n, int k, int epilogue) {
     return epilogue == kEpiSwiGLU && m <= 64 && n % 64 == 0 && ((k + 31) / 32) % 4 == 0;
 }
+
+// At most kFewRows rows: gemm_few_rows_kernel, K split over workgroups as far
+// as one pass over the CUs goes (single TinyLlama step: 128 workgroups for O
+// and down 0.7 us more per product, two passes of splits 2 us more).
+static bool few_rows(int m, int n, int epilogue) { return m <= kFewRows && (epilogue == kEpiStore || n % 64 == 0); }
 
 struct GemmChoice {
     GemmCfg cfg;
@@ -712,6 +855,19 @@ static GemmChoice choose_tiles(int m, int n, int k, int epilogue) {
 
 GemmPlan gemm_plan(int m, int n, int k, int epilogue) {
     GemmPlan p;
+    if (few_rows(m, n, epilogue)) {
+        p.few_rows = true;
+        p.KT = (k + 31) / 32;
+        p.NT = (n + 31) / 32;
+        p.row_blocks = 1;
+        p.col_blocks = epilogue == kEpiSwiGLU ? n / 32 : (n + 15) / 16;
+        const int splits = epilogue == kEpiSwiGLU ? 1 : std::max(1, std::min(device_cus() / p.col_blocks, p.KT / 32));
+        p.kt_per_split = (p.KT + splits - 1) / splits;
+        p.splits = (p.KT + p.kt_per_split - 1) / p.kt_per_split;
+        p.direct = p.splits == 1;
+        p.ws_floats = p.direct ? 0 : (size_t)p.splits * m * n;
+        return p;
+    }
     if (swiglu_ksplit(m, n, k, epilogue)) {
         p.KT = (k + 31) / 32;
         p.NT = (n + 31) / 32;
@@ -747,6 +903,20 @@ static void gemm_launch(const GemmPlan& p, hipStream_t stream, const uint16_t* a
                        p.kt_per_split, p.splits, p.row_blocks, p.col_blocks, split_stride, h, h_lo);
 }
 
+template <int NW, int U, int HL, int SWIGLU>
+static void few_rows_launch(const GemmPlan& p, hipStream_t stream, const uint16_t* a, int m, const uint16_t* w,
+                            float* c, int n, size_t split_stride, uint16_t* h) {
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(p.col_blocks * p.splits)), dim3(NW * 64), 0, stream, a, m, w,
+                           p.KT, p.NT, c, n, p.kt_per_split, p.splits, split_stride, h);
+    };
+    static_assert(kFewRows == 8, "row counts below");
+    if (m == 1) go(gemm_few_rows_kernel<1, NW, U, HL, SWIGLU>);
+    else if (m == 2) go(gemm_few_rows_kernel<2, NW, U, HL, SWIGLU>);
+    else if (m <= 4) go(gemm_few_rows_kernel<4, NW, U, HL, SWIGLU>);
+    else go(gemm_few_rows_kernel<8, NW, U, HL, SWIGLU>);
+}
+
 zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_packed, float* c_f32,
                       uint16_t* c_bf16, int m, int n, int k, int epilogue, Slabs* deferred) {
     if (deferred && (epilogue != kEpiStore || !c_f32 || c_bf16))
@@ -758,11 +928,22 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
     if (a_bytes > 0x7fffffffull || w_bytes > 0x7fffffffull)
         return set_err(ctx, ZR_E_UNSUPPORTED, "GEMM operands of %zu / %zu bytes exceed 2 GiB", a_bytes, w_bytes);
     const bool split_act = (ctx->desc.flags & ZR_FLAG_SPLIT_ACTIVATIONS) != 0;
-    if (swiglu_ksplit(m, n, k, epilogue) && (!c_bf16 || c_f32 || deferred))
+    const GemmPlan p = gemm_plan(m, n, k, epilogue);
+    const bool in_launch = p.few_rows ? epilogue == kEpiSwiGLU : swiglu_ksplit(m, n, k, epilogue);
+    if (in_launch && (!c_bf16 || c_f32 || deferred))
         return set_err(ctx, ZR_E_INVARIANT, "K-split SwiGLU (M=%d) writes the bf16 operand only", m);
-    if (swiglu_ksplit(m, n, k, epilogue)) {
-        const GemmPlan p = gemm_plan(m, n, k, epilogue);
-        hipEvent_t ev;
+    hipEvent_t ev;
+    if (in_launch && p.few_rows) {
+        timing_mark_begin(ctx, kClassGemm, &ev);
+        if (split_act)
+            few_rows_launch<4, 2, 2, 1>(p, ctx->stream, a, m, w_packed, nullptr, n, 0, c_bf16);
+        else
+            few_rows_launch<4, 2, 1, 1>(p, ctx->stream, a, m, w_packed, nullptr, n, 0, c_bf16);
+        ZR_LAUNCH_CHECK(ctx);
+        timing_mark_end(ctx, kClassGemm, ev);
+        return ZR_OK;
+    }
+    if (in_launch) {
         timing_mark_begin(ctx, kClassGemm, &ev);
 #define ZR_KSPLIT(HLV, MTV)                                                                                     \
     hipLaunchKernelGGL((gemm_swiglu_ksplit_kernel<3, HLV, MTV>), dim3(p.col_blocks), dim3(256), 0, ctx->stream, a, \
@@ -783,7 +964,6 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
         timing_mark_end(ctx, kClassGemm, ev);
         return ZR_OK;
     }
-    const GemmPlan p = gemm_plan(m, n, k, epilogue);
     if (swiglu_fused(m, epilogue) && (!c_bf16 || c_f32 || n % 64 != 0))
         return set_err(ctx, ZR_E_INVARIANT, "fused SwiGLU writes the bf16 operand only (N=%d)", n);
     const bool fused = swiglu_fused(m, epilogue);
@@ -792,9 +972,15 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
     if (!direct && (size_t)p.splits * split_stride > ctx->splitk_ws_floats)
         return set_err(ctx, ZR_E_OOM, "split-K workspace too small (%d x %d x %d)", p.splits, m, n);
     float* dst = direct ? c_f32 : ctx->splitk_ws;
-    hipEvent_t ev;
     timing_mark_begin(ctx, kClassGemm, &ev);
     bool launched = false;
+    if (p.few_rows) {
+        if (split_act)
+            few_rows_launch<4, 4, 2, 0>(p, ctx->stream, a, m, w_packed, dst, n, split_stride, nullptr);
+        else
+            few_rows_launch<4, 4, 1, 0>(p, ctx->stream, a, m, w_packed, dst, n, split_stride, nullptr);
+        launched = true;
+    }
 #define ZR_GEMM_FUSED_CASE(WMV, WNV, WAM, WAN, ST)                                                     \
     if (fused && !launched && p.wm == WMV && p.wn == WNV && p.waves_m == WAM && p.waves_n == WAN &&    \
         p.stages == ST) {                                                                              \

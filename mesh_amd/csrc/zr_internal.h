@@ -429,6 +429,7 @@ zr_status launch_sample(zr_context* ctx, const float* d_logits, int rows, int co
 enum GemmEpilogue { kEpiStore = 0, kEpiSwiGLU = 1 };
 struct GemmPlan {
     int wm = 0, wn = 0, waves_m = 0, waves_n = 0, stages = 0;  // tile configuration
+    bool few_rows = false;                                     // gemm_few_rows_kernel instead
     int KT = 0, NT = 0, row_blocks = 0, col_blocks = 0, splits = 1, kt_per_split = 0;
     bool direct = true;
     size_t ws_floats = 0;
