@@ -454,10 +454,17 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     // split's append then add little to a split (256 Llama-3 sessions, ~96
     // pages per split: 17.9 -> 17.3 ms per step), where 8- to 12-page splits
     // (32 TinyLlama sessions) lose more than the RoPE launch costs
-    // (1.49 -> 1.59 ms).  ZR_ATTN_FUSE_ROPE=1 / 0 forces either path.
+    // (1.49 -> 1.59 ms).  It also does so when the QKV product leaves at most
+    // two slabs to sum (steps of at most 8 rows; one TinyLlama session: the
+    // attention launch 6.9 -> 7.7 us, the RoPE launch's 2.9 saved).
+    // ZR_ATTN_FUSE_ROPE=1 / 0 forces either path.
     st->pure_decode = !ctx->plain_kv && S > 0 && st->n_pblocks == 0;
     for (int s = 0; s < S && st->pure_decode; ++s) st->pure_decode = mb->q_len[s] == 1;
     st->fuse_rope = st->pure_decode && pps >= 48;
+    if (st->pure_decode && !st->fuse_rope) {
+        const GemmPlan qkv = gemm_plan(total_q, ctx->q_cols + 2 * ctx->kv_cols, ctx->desc.hidden, kEpiStore);
+        st->fuse_rope = qkv.few_rows && qkv.splits <= 2;
+    }
     if (const char* env = getenv("ZR_ATTN_FUSE_ROPE")) st->fuse_rope = st->pure_decode && atoi(env) != 0;
     st->grid_items = st->n_attn_items;
     st->grid_merge = st->n_merge;
