@@ -783,8 +783,11 @@ zr_status zr_context_create(const zr_model_desc* desc, int device, zr_context** 
         delete ctx;
         return src;
     }
-    e = hipHostMalloc((void**)&ctx->h_token_err, sizeof(unsigned long long), hipHostMallocDefault);
+    // pinned: the token check word, then the sampler's parameters
+    ctx->sample_ws_bytes = kSampleArgBytes * (size_t)std::max(d.max_seqs, 512);
+    e = hipHostMalloc((void**)&ctx->h_token_err, 64 + ctx->sample_ws_bytes, hipHostMallocDefault);
     if (e != hipSuccess) return fail(e, "hipHostMalloc token check word");
+    ctx->sample_ws = (unsigned char*)ctx->h_token_err + 64;
     *ctx->h_token_err = ~0ull;
     e = hipMemcpy(ctx->d_token_err, ctx->h_token_err, sizeof(unsigned long long), hipMemcpyHostToDevice);
     if (e != hipSuccess) return fail(e, "hipMemcpy token check word");
@@ -812,7 +815,7 @@ void zr_context_destroy(zr_context* ctx) {
     if (ctx->kv_stage) (void)hipFree(ctx->kv_stage);
     if (ctx->cbor_ws) (void)hipFree(ctx->cbor_ws);
     if (ctx->cbor_out) (void)hipFree(ctx->cbor_out);
-    if (ctx->sample_ws) (void)hipFree(ctx->sample_ws);
+    if (ctx->sample_ws_own) (void)hipHostFree(ctx->sample_ws_own);
     free_ctx_buffers(ctx);
     destroy_streams(ctx);
     delete ctx;

@@ -247,8 +247,9 @@ struct zr_context {
     size_t cbor_ws_bytes = 0;
     void* cbor_out = nullptr;       // KV snapshot encoder / decoder: the document on the device
     size_t cbor_out_bytes = 0;
-    void* sample_ws = nullptr;      // stochastic sampling: per-row parameters
+    void* sample_ws = nullptr;      // stochastic sampling: per-row parameters (pinned host memory)
     size_t sample_ws_bytes = 0;
+    void* sample_ws_own = nullptr;  // ... of calls with more rows than the context's own block holds
     // Device-fed token ids out of the vocabulary: the embedding kernel keeps
     // the smallest (row << 32 | id) here (all ones = none); a forward pass fed
     // from device memory copies it to the pinned host word, which
@@ -422,6 +423,7 @@ constexpr int kNoAllocArgmaxPairs = 32768;
 constexpr int kMaxDevices = 64;
 zr_status noalloc_scratch_init(zr_context* ctx);
 zr_status launch_argmax_noalloc(zr_context* ctx, const float* x, int rows, int cols, uint32_t* out);
+constexpr size_t kSampleArgBytes = 32;  // per-row parameters of launch_sample
 // sample_tokens_device_with_seeds per row (sample.hip); parameters are host arrays
 zr_status launch_sample(zr_context* ctx, const float* d_logits, int rows, int cols, const float* temperature,
                         const float* top_p, const uint64_t* seeds, uint32_t* d_out);
