@@ -106,7 +106,7 @@ static zr_status resolve_geometry(zr_context* ctx) {
         ctx->kv_head_map.push_back((uint32_t)(gk - ctx->kv_head_start));
     }
     // RoPE's rotate-half pairs dims (i, i + d / 2): an even head_dim
-    // (tensor_ops.rs:509-520); the generic attention kernel holds up to 256
+    // (tensor_ops.rs:509-520); the plain-layout attention kernels hold up to 256
     // dims per lane group
     if (head_dim % 2 != 0 || head_dim > 256)
         return set_err(ctx, ZR_E_UNSUPPORTED, "head_dim %d not supported (even, at most 256)", head_dim);

@@ -184,7 +184,7 @@ struct zr_context {
     // decode / prefill attention kernels (head_dim 64 or 128, q heads per kv
     // head dividing 16).  true (any other even head_dim up to 256, any group):
     // each kv head's K and V tiles are row-major [16 rows][head_dim], read by
-    // the generic attention kernel.
+    // the plain-layout attention kernels.
     bool plain_kv = false;
 
     // weights
