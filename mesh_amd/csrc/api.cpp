@@ -131,7 +131,7 @@ static void destroy_streams(zr_context* ctx) {
 }
 
 static void free_ctx_buffers(zr_context* ctx) {
-    void* bufs[] = {ctx->hidden, ctx->xa, ctx->qkv, ctx->q_rope, ctx->attn_a, ctx->proj, ctx->ffn_a,
+    void* bufs[] = {ctx->hidden, ctx->hidden2, ctx->xa, ctx->qkv, ctx->q_rope, ctx->attn_a, ctx->proj, ctx->ffn_a,
                     ctx->logits, ctx->final_a, ctx->tokens_out, ctx->splitk_ws, ctx->attn_part,
                     ctx->argmax_ws, ctx->inv_freq, ctx->kv_pool, ctx->embedding, ctx->lm_head,
                     ctx->final_norm, ctx->d_token_err};
@@ -585,15 +585,28 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
     // split-K products are left as slabs for the next kernel to sum, except
     // where the caller asked for the per-layer partials (those are copied out)
     Slabs down(nullptr);
+    // one or two rows: the norms inside the products that read them, the
+    // residual stream alternating between two buffers
+    const bool norm_qkv = norm_in_gemm(T, QKV, H, kEpiStore);
+    const bool norm_gate_up = norm_in_gemm(T, 2 * F, H, kEpiSwiGLU);
+    float *hidden = ctx->hidden, *other = ctx->hidden2;
     for (int l = 0; l < d.num_layers; ++l) {
         const LayerDev& L = ctx->layers[l];
         Slabs* defer = h_partials ? nullptr : &down;
         // hidden += previous down partial; xa = rms_norm(hidden) * attn_norm
-        if ((rc = launch_rms_norm(ctx, ctx->hidden, l > 0 ? down : Slabs(nullptr), ctx->hidden, L.attn_norm, nullptr,
-                                  ctx->xa, lo, nullptr, T, H)))
-            return rc;
         Slabs qkv(ctx->qkv);
-        if ((rc = launch_gemm(ctx, ctx->xa, L.w_qkv, ctx->qkv, nullptr, T, QKV, H, kEpiStore, &qkv))) return rc;
+        if (norm_qkv) {
+            const Slabs res = l > 0 ? down : Slabs(nullptr);
+            if ((rc = launch_norm_gemm(ctx, hidden, res, other, L.attn_norm, L.w_qkv, ctx->qkv, nullptr, T, QKV, H,
+                                       kEpiStore)))
+                return rc;
+            if (res.ptr) std::swap(hidden, other);
+        } else {
+            if ((rc = launch_rms_norm(ctx, hidden, l > 0 ? down : Slabs(nullptr), hidden, L.attn_norm, nullptr,
+                                      ctx->xa, lo, nullptr, T, H)))
+                return rc;
+            if ((rc = launch_gemm(ctx, ctx->xa, L.w_qkv, ctx->qkv, nullptr, T, QKV, H, kEpiStore, &qkv))) return rc;
+        }
         if (st->fuse_rope) {  // RoPE + KV append inside the decode attention launch
             if ((rc = launch_attention_rope(ctx, st, l, qkv, 1, nullptr, ctx->attn_a))) return rc;
         } else {
@@ -608,10 +621,17 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
             ZR_HIP(ctx, hipMemcpyAsync(h_partials + ((size_t)l * 2 + 0) * T * H, ctx->proj, sizeof(float) * T * H,
                                        hipMemcpyDeviceToHost, ctx->stream));
         // post_attn = hidden + o_partial (identity all-reduce at one worker)
-        if ((rc = launch_rms_norm(ctx, ctx->hidden, o, ctx->hidden, L.mlp_norm, nullptr, ctx->xa, lo, nullptr,
-                                  T, H)))
-            return rc;
-        if ((rc = launch_gemm(ctx, ctx->xa, L.w_gate_up, nullptr, ctx->ffn_a, T, 2 * F, H, kEpiSwiGLU))) return rc;
+        if (norm_gate_up) {
+            if ((rc = launch_norm_gemm(ctx, hidden, o, other, L.mlp_norm, L.w_gate_up, nullptr, ctx->ffn_a, T, 2 * F,
+                                       H, kEpiSwiGLU)))
+                return rc;
+            std::swap(hidden, other);
+        } else {
+            if ((rc = launch_rms_norm(ctx, hidden, o, hidden, L.mlp_norm, nullptr, ctx->xa, lo, nullptr, T, H)))
+                return rc;
+            if ((rc = launch_gemm(ctx, ctx->xa, L.w_gate_up, nullptr, ctx->ffn_a, T, 2 * F, H, kEpiSwiGLU)))
+                return rc;
+        }
         down = Slabs(ctx->proj);
         if ((rc = launch_gemm(ctx, ctx->ffn_a, L.w_down, ctx->proj, nullptr, T, H, F, kEpiStore, defer))) return rc;
         if (h_partials)
@@ -619,7 +639,7 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
                                        hipMemcpyDeviceToHost, ctx->stream));
     }
     // final residual + norm on the last row of every sequence, LM head, argmax
-    if ((rc = launch_rms_norm(ctx, ctx->hidden, down, ctx->hidden, ctx->final_norm, nullptr, ctx->final_a, lo,
+    if ((rc = launch_rms_norm(ctx, hidden, down, hidden, ctx->final_norm, nullptr, ctx->final_a, lo,
                               st->last_rows, S, H)))
         return rc;
     float* logits = ctx->logits;
@@ -734,6 +754,7 @@ zr_status zr_context_create(const zr_model_desc* desc, int device, zr_context** 
         size_t bytes;
     } allocs[] = {
         {(void**)&ctx->hidden, 4 * T * H},
+        {(void**)&ctx->hidden2, 4 * std::min<size_t>(T, kNormRows) * H},
         {(void**)&ctx->xa, 2 * 2 * a_plane((int)T, (int)H)},
         {(void**)&ctx->qkv, 4 * T * (Q + 2 * KV)},   {(void**)&ctx->q_rope, 4 * T * Q},
         {(void**)&ctx->attn_a, 2 * 2 * a_plane((int)T, (int)Q)},

@@ -345,7 +345,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(
     }
 }
 
-// gate/up + SwiGLU for at most 32 rows in one launch: K split over the 4
+// gate/up + SwiGLU for 9-32 rows (33-64: MT = 2) in one launch: K split over the 4
 // waves of a workgroup instead of over workgroups (no slabs, no reduce
 // kernel).  A workgroup owns one gate / up tile pair (64 columns of the
 // interleaved product, 32 columns of H); wave w takes k-steps w, w + 4, ...
@@ -505,17 +505,40 @@ __global__ __launch_bounds__(256) void gemm_swiglu_ksplit_kernel(const uint16_t*
 // sessions 621 / 656 us per step of 4 layers).
 constexpr int kFewRows = 8;
 constexpr int kWeightCache = 2;  // nontemporal: read once per product
-template <int MR, int NW, int U, int HL, int SWIGLU>
+struct NormRows {
+    const float *x, *res;
+    int res_n;
+    size_t res_stride;
+    float* x_out;
+    const float* gamma;
+    float eps;
+};
+// block barrier for LDS data that leaves loads to registers in flight
+__device__ __forceinline__ void lds_barrier() {
+    wave_copies_wait<63>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// NORM: A is rms_norm(x + residual) gamma (launch_norm_gemm): every workgroup
+// reads the rows, their residual slabs and gamma (L2 hits, under its first
+// weights' flight), normalises them as the norm kernel does and keeps them in
+// LDS; workgroup 0 writes x + residual to x_out (another buffer: the rest still
+// read x).  TinyLlama, one row: gate/up 11.9 us with or without, QKV 5.0 -> 5.8,
+// and no norm launches of 3.6; the step 1.07 -> 0.95 ms.
+template <int MR, int NW, int U, int HL, int SWIGLU, int NORM>
 __global__ __launch_bounds__(NW * 64) void gemm_few_rows_kernel(const uint16_t* __restrict__ A, int M,
                                                                 const uint16_t* __restrict__ Wp, int KT, int NT,
                                                                 float* __restrict__ C, int N, int kt_per_split,
                                                                 int splits, size_t split_stride,
-                                                                uint16_t* __restrict__ H) {
+                                                                uint16_t* __restrict__ H, NormRows nr) {
     constexpr int TW = SWIGLU ? 2 : 1;
     constexpr int NA = (U * HL * 4 * MR + 63) / 64;  // loads of A runs per set
     typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
     __shared__ f32x4 red[NW][TW][64];
-    __shared__ u32x4 rows[NW][NA * 64];  // [step u][hi, lo][q][row]
+    __shared__ u32x4 rows[NORM ? 1 : NW][NORM ? 1 : NA * 64];  // [step u][hi, lo][q][row]
+    extern __shared__ bf16x8 normed[];                         // NORM: [k / 8][hi, lo][row]
+    constexpr int KC = kNormCols / (8 * NW * 64);              // runs of 8 columns per thread
+    f32x4 xv[MR][KC][2], gv[KC][2];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int col16 = blockIdx.x / splits, split = blockIdx.x - col16 * splits;
     const int q = lane >> 4, i16 = lane & 15;
@@ -546,7 +569,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_rows_kernel(const uint16_t* 
     u32x4 wr[2][U][TW], ar[2][NA];
     auto load = [&](int set, int s) {
 #pragma unroll
-        for (int v = 0; v < NA; ++v)
+        for (int v = 0; v < (NORM ? 0 : NA); ++v)
             ar[set][v] = __builtin_amdgcn_raw_buffer_load_b128(
                 rsrc_a, (int)(s + au[v] < s1 ? a0[v] + ((unsigned)s << 11) : kPast), 0, 0);
 #pragma unroll
@@ -560,35 +583,114 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_rows_kernel(const uint16_t* 
     f32x4 acc[TW];
 #pragma unroll
     for (int t = 0; t < TW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto products = [&](int set) {
-        // (one wave's LDS operations run in order; the fences keep the compiler's order the same)
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+    auto products = [&](int set, int s) {
+        if constexpr (!NORM) {
+            // (one wave's LDS operations run in order; the fences keep the compiler's order the same)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int v = 0; v < NA; ++v) rows[wave][v * 64 + lane] = ar[set][v];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+            for (int v = 0; v < NA; ++v) rows[wave][v * 64 + lane] = ar[set][v];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int h = 0; h < HL; ++h) {
-                const bf16x8 fa =
-                    __builtin_bit_cast(bf16x8, rows[wave][((u * HL + h) * 4 + q) * MR + (i16 & (MR - 1))]);
+                bf16x8 fa;
+                if constexpr (NORM)  // (a step past the wave's run repeats its last: its weights are zeros)
+                    fa = normed[((min(s + u, s1 - 1) * 4 + q) * HL + h) * MR + (i16 & (MR - 1))];
+                else
+                    fa = __builtin_bit_cast(bf16x8, rows[wave][((u * HL + h) * 4 + q) * MR + (i16 & (MR - 1))]);
 #pragma unroll
                 for (int t = 0; t < TW; ++t)
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, __builtin_bit_cast(bf16x8, wr[set][u][t]),
                                                                      acc[t], 0, 0, 0);
             }
     };
+    const int chunks = KT * 4;  // runs of 8 columns
+    f32x4 rv[MR][KC][2][2];
+    if constexpr (NORM) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int ch = tid + k * NW * 64;
+            const bool in = ch < chunks;
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                gv[k][p] = in ? *(const f32x4*)(nr.gamma + ch * 8 + 4 * p) : zero;
+#pragma unroll
+                for (int r = 0; r < MR; ++r) {
+                    const size_t at = (size_t)r * KT * 32 + ch * 8 + 4 * p;
+                    const bool ok = in && r < M;
+                    xv[r][k][p] = ok ? *(const f32x4*)(nr.x + at) : zero;
+#pragma unroll
+                    for (int n2 = 0; n2 < 2; ++n2)
+                        rv[r][k][p][n2] =
+                            ok && n2 < nr.res_n ? *(const f32x4*)(nr.res + n2 * nr.res_stride + at) : zero;
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     load(0, s0);
+    if constexpr (NORM) {
+        __builtin_amdgcn_sched_barrier(0);
+        __shared__ float ssum[MR][NW];
+#pragma unroll
+        for (int r = 0; r < MR; ++r) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int k = 0; k < KC; ++k) {
+                const int ch = tid + k * NW * 64;
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const size_t at = (size_t)r * KT * 32 + ch * 8 + 4 * p;
+                    if (nr.res_n > 0) {
+                        f32x4 sum = rv[r][k][p][0];
+                        if (nr.res_n > 1) sum += rv[r][k][p][1];
+                        for (int n2 = 2; n2 < nr.res_n; ++n2)
+                            if (ch < chunks && r < M) sum += *(const f32x4*)(nr.res + n2 * nr.res_stride + at);
+                        xv[r][k][p] += sum;
+                        if (blockIdx.x == 0 && ch < chunks && r < M) *(f32x4*)(nr.x_out + at) = xv[r][k][p];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ss += xv[r][k][p][e] * xv[r][k][p][e];
+                }
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+            if (lane == 0) ssum[r][wave] = ss;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int r = 0; r < MR; ++r) {
+            float total = 0.0f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) total += ssum[r][w];
+            const float inv = 1.0f / sqrtf(total / (float)(KT * 32) + nr.eps);
+#pragma unroll
+            for (int k = 0; k < KC; ++k) {
+                const int ch = tid + k * NW * 64;
+                float y[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) y[e] = xv[r][k][e >> 2][e & 3] * inv * gv[k][e >> 2][e & 3];
+                if (ch < chunks) {
+                    normed[(ch * HL + 0) * MR + r] = to_bf16x8(y, false);
+                    if (HL == 2) normed[(ch * HL + HL - 1) * MR + r] = to_bf16x8(y, true);
+                }
+            }
+        }
+        lds_barrier();
+    }
     for (int s = s0; s < s1; s += 2 * U) {
         load(1, s + U);
         __builtin_amdgcn_sched_barrier(0);
-        products(0);
+        products(0, s);
         __builtin_amdgcn_sched_barrier(0);
         load(0, s + 2 * U);
         __builtin_amdgcn_sched_barrier(0);
-        products(1);
+        products(1, s + U);
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -905,16 +1007,61 @@ static void gemm_launch(const GemmPlan& p, hipStream_t stream, const uint16_t* a
 
 template <int NW, int U, int HL, int SWIGLU>
 static void few_rows_launch(const GemmPlan& p, hipStream_t stream, const uint16_t* a, int m, const uint16_t* w,
-                            float* c, int n, size_t split_stride, uint16_t* h) {
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(p.col_blocks * p.splits)), dim3(NW * 64), 0, stream, a, m, w,
-                           p.KT, p.NT, c, n, p.kt_per_split, p.splits, split_stride, h);
+                            float* c, int n, size_t split_stride, uint16_t* h, const NormRows* nr = nullptr) {
+    auto go = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(p.col_blocks * p.splits)), dim3(NW * 64), lds, stream, a, m, w,
+                           p.KT, p.NT, c, n, p.kt_per_split, p.splits, split_stride, h, nr ? *nr : NormRows{});
     };
-    static_assert(kFewRows == 8, "row counts below");
-    if (m == 1) go(gemm_few_rows_kernel<1, NW, U, HL, SWIGLU>);
-    else if (m == 2) go(gemm_few_rows_kernel<2, NW, U, HL, SWIGLU>);
-    else if (m <= 4) go(gemm_few_rows_kernel<4, NW, U, HL, SWIGLU>);
-    else go(gemm_few_rows_kernel<8, NW, U, HL, SWIGLU>);
+    static_assert(kFewRows == 8 && kNormRows == 2, "row counts below");
+    if (nr) {
+        if (m == 1) go(gemm_few_rows_kernel<1, NW, U, HL, SWIGLU, 1>, (size_t)p.KT * 64 * HL);
+        else go(gemm_few_rows_kernel<2, NW, U, HL, SWIGLU, 1>, (size_t)p.KT * 128 * HL);
+        return;
+    }
+    if (m == 1) go(gemm_few_rows_kernel<1, NW, U, HL, SWIGLU, 0>, 0);
+    else if (m == 2) go(gemm_few_rows_kernel<2, NW, U, HL, SWIGLU, 0>, 0);
+    else if (m <= 4) go(gemm_few_rows_kernel<4, NW, U, HL, SWIGLU, 0>, 0);
+    else go(gemm_few_rows_kernel<8, NW, U, HL, SWIGLU, 0>, 0);
+}
+
+// Every workgroup normalises the rows for itself, from L2 and under the flight
+// of its first weights: one or two rows cost a product 0-0.8 us where the norm
+// launch took 3.6, until the rows read again weigh beside the weights (Llama-3
+// gate/up, 1792 workgroups of 16 KB per row and buffer: step of 4 layers with
+// one row 675 -> 659 us, with two 479 -> 492).
+bool norm_in_gemm(int m, int n, int k, int epilogue) {
+    if (m < 1 || m > kNormRows || k > kNormCols || k % 32 != 0 || !few_rows(m, n, epilogue) ||
+        2 * packed_weight_elems(k, n) > 0x7fffffffull)
+        return false;
+    const GemmPlan p = gemm_plan(m, n, k, epilogue);
+    return p.direct && m * p.col_blocks <= 2048;
+}
+
+zr_status launch_norm_gemm(zr_context* ctx, const float* x, const Slabs& residual, float* x_out, const float* gamma,
+                           const uint16_t* w_packed, float* c_f32, uint16_t* c_bf16, int m, int n, int k,
+                           int epilogue) {
+    if (!norm_in_gemm(m, n, k, epilogue) || x_out == x || (epilogue == kEpiSwiGLU ? !c_bf16 : !c_f32))
+        return set_err(ctx, ZR_E_INVARIANT, "no normalising product for %d x %d x %d", m, n, k);
+    const GemmPlan p = gemm_plan(m, n, k, epilogue);
+    const bool split_act = (ctx->desc.flags & ZR_FLAG_SPLIT_ACTIVATIONS) != 0;
+    const NormRows nr = {x, residual.ptr, residual.ptr ? residual.n : 0, residual.stride, x_out, gamma,
+                         ctx->desc.rms_norm_eps};
+    hipEvent_t ev;
+    timing_mark_begin(ctx, kClassGemm, &ev);
+    if (epilogue == kEpiSwiGLU) {
+        if (split_act)
+            few_rows_launch<4, 2, 2, 1>(p, ctx->stream, nullptr, m, w_packed, nullptr, n, 0, c_bf16, &nr);
+        else
+            few_rows_launch<4, 2, 1, 1>(p, ctx->stream, nullptr, m, w_packed, nullptr, n, 0, c_bf16, &nr);
+    } else {
+        if (split_act)
+            few_rows_launch<4, 4, 2, 0>(p, ctx->stream, nullptr, m, w_packed, c_f32, n, 0, nullptr, &nr);
+        else
+            few_rows_launch<4, 4, 1, 0>(p, ctx->stream, nullptr, m, w_packed, c_f32, n, 0, nullptr, &nr);
+    }
+    ZR_LAUNCH_CHECK(ctx);
+    timing_mark_end(ctx, kClassGemm, ev);
+    return ZR_OK;
 }
 
 zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_packed, float* c_f32,

@@ -203,6 +203,7 @@ struct zr_context {
     // activations (max_tokens rows).  GEMM A operands are bf16 [M, K], followed
     // by the lo half [M, K] under ZR_FLAG_SPLIT_ACTIVATIONS.
     float* hidden = nullptr;     // [T, H] residual stream (f32)
+    float* hidden2 = nullptr;    // [kNormRows, H] its other buffer (launch_norm_gemm)
     uint16_t* xa = nullptr;      // normed hidden, A of QKV / gate_up
     float* qkv = nullptr;        // [T, Q + 2Kc]
     float* q_rope = nullptr;     // [T, Q]
@@ -444,6 +445,14 @@ GemmPlan gemm_plan(int m, int n, int k, int epilogue);
 // *deferred then describes C either way.
 zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_packed, float* c_f32,
                       uint16_t* c_bf16, int m, int n, int k, int epilogue, Slabs* deferred = nullptr);
+constexpr int kNormRows = 2, kNormCols = 4096;  // the most rows / columns normalised inside a product
+// The product of rms_norm(x + residual) gamma in one launch, for the few rows
+// norm_in_gemm takes (its plan has no split-K slabs: the residual's may lie in
+// that workspace).  With a residual, x + residual goes to x_out (not x).
+bool norm_in_gemm(int m, int n, int k, int epilogue);
+zr_status launch_norm_gemm(zr_context* ctx, const float* x, const Slabs& residual, float* x_out, const float* gamma,
+                           const uint16_t* w_packed, float* c_f32, uint16_t* c_bf16, int m, int n, int k,
+                           int epilogue);
 // f32 [rows, K] -> fragment-packed bf16 hi (+ lo) A operand (K % 32 == 0)
 zr_status launch_to_bf16_pair(zr_context* ctx, const float* x, int rows, int K, uint16_t* out, int with_lo);
 // fragment-packed bf16 hi (+ lo) [rows, K] -> f32 hi + lo [rows, K]
