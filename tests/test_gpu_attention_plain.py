@@ -1,6 +1,7 @@
-"""Attention over plain-layout pools (attention_plain.hip: head_dim a multiple
-of 4 other than 64 / 128, or q heads per kv head not dividing 16) against a
-float64 restatement.
+"""Attention over plain-layout pools (head_dim other than 64 / 128, or q heads
+per kv head not dividing 16) against a float64 restatement: column tiles for a
+head_dim that is a multiple of 4 (attention_plain.hip), one wave per row and q
+head for the others (attention.hip's paged_attention_generic_kernel).
 
 Tolerance: every product and sum is f32, as in the reference; a score of D
 products and a weighted sum of L values carry a few rounding errors of 2^-24 of
@@ -90,6 +91,20 @@ def test_every_multiple_of_four_head_dim_and_group(kv_dtype, heads, kv_heads, D)
     windows; head dims on both sides of every block of 16 and group of 64; 1
     to 32 q heads per kv head."""
     cases = [(0, 1, 0), (0, 37, 0), (300, 1, 0), (57, 20, 9), (16, 1, 0), (130, 1, 5)]
+    out, seqs = run_attention(heads, kv_heads, D, kv_dtype, cases, np.random.default_rng(D * heads + kv_heads))
+    want = reference(seqs, heads, kv_heads, D)
+    err = np.abs(out - want).reshape(len(out), heads, D).max(-1) / np.abs(want).reshape(len(out), heads, D).max(-1)
+    assert err.max() <= RTOL, np.unravel_index(err.argmax(), err.shape)
+
+
+@pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("heads,kv_heads,D", [(16, 16, 2), (16, 4, 6), (48, 16, 18), (16, 2, 62), (16, 16, 66),
+                                              (16, 2, 98), (16, 8, 126), (16, 16, 130), (16, 4, 190), (16, 2, 254)])
+def test_even_head_dims_that_are_no_multiple_of_four(kv_dtype, heads, kv_heads, D):
+    """The scalar kernel: a wave walks 64 keys at a time and holds up to 4 dims
+    a lane, so windows end inside the first 64 keys, on the 64th and past it,
+    and head dims on both sides of 64, 128 and 192."""
+    cases = [(0, 1, 0), (0, 37, 0), (300, 1, 0), (57, 20, 9), (63, 2, 0), (130, 1, 5)]
     out, seqs = run_attention(heads, kv_heads, D, kv_dtype, cases, np.random.default_rng(D * heads + kv_heads))
     want = reference(seqs, heads, kv_heads, D)
     err = np.abs(out - want).reshape(len(out), heads, D).max(-1) / np.abs(want).reshape(len(out), heads, D).max(-1)

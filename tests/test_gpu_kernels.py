@@ -896,7 +896,7 @@ def test_c5_shape_attention_256_sessions_matches_oracle(rope, kv_dtype):
 @pytest.mark.parametrize("heads,kv_heads,D", [(8, 2, 96), (6, 2, 16), (12, 4, 64)])
 def test_generic_attention_and_plain_pages(kv_dtype, heads, kv_heads, D):
     """Head dims 96 and 16, and 3 q heads per kv head at D = 64: pages in the
-    plain layout, attention by the generic kernel.  Decode rows and causal
+    plain layout, attention by its column tiles.  Decode rows and causal
     chunks over imported prefixes (one trimmed to start mid-page) against the
     oracle within 2e-3; the pages round-trip bit for bit through export /
     import."""

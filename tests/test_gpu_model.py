@@ -450,9 +450,21 @@ def test_reference_test_model_sliding_window_decode_kat():
 @pytest.mark.parametrize("hidden,heads,kv_heads", [(256, 16, 4), (384, 4, 2), (512, 16, 16), (576, 9, 3)])
 def test_generic_head_dim_models_match_oracle(kv_dtype, hidden, heads, kv_heads):
     """Head dims 16, 96, 32 and a 64-dim model whose 3 q heads per kv head do
-    not divide 16: the plain page layout and the generic attention kernel.
+    not divide 16: the plain page layout and its column-tile attention.
     Prompts of 1 to 40 tokens (prefill chunks with causal masking), then
     decode microbatches."""
+    plain_layout_model(kv_dtype, hidden, heads, kv_heads)
+
+
+@pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("hidden,heads,kv_heads", [(160, 16, 16), (576, 32, 16)])
+def test_models_of_head_dims_that_are_no_multiple_of_four(kv_dtype, hidden, heads, kv_heads):
+    """Head dims 10 and 18: the same steps on the scalar attention kernel, whose
+    output goes out as the O product's bf16 hi + lo operand."""
+    plain_layout_model(kv_dtype, hidden, heads, kv_heads)
+
+
+def plain_layout_model(kv_dtype, hidden, heads, kv_heads):
     cfg = dict(hidden=hidden, num_heads=heads, num_kv_heads=kv_heads, num_layers=2, vocab=300, ffn=512,
                rms_norm_eps=1e-5, rope_base=10000.0)
     geo = geometry(cfg)
