@@ -762,8 +762,7 @@ def test_gemm_matches_fp64(split, m, k, n):
                                    (40, 512, 512), (33, 256, 96),  # 33-64 rows: K over 4 waves, two row tiles
                                    (64, 4096, 7168),     # the tensor-parallel shard's gate / up at 64 sessions
                                    (32, 2048, 5632),     # the 32-session TinyLlama gate / up: K over 4 waves
-                                   (1, 128, 64), (7, 256, 96),  # <= 32 rows, K over 4 waves of 1 / 2 steps
-                                   (5, 96, 64),          # K = 3 steps: split-K slabs and the reduce
+                                   (1, 128, 64), (7, 256, 96), (5, 96, 64),  # at most 8 rows: weights to registers
                                    (100, 256, 512),      # 65-128 rows: fused, 64 x 256 tiles
                                    (130, 200, 96),       # fused, 128 x 256 tiles, K padded to 224
                                    (256, 4096, 14336),   # the Llama-3-8B gate / up product of the decode step
