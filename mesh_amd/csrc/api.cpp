@@ -573,7 +573,7 @@ static zr_status check_ready(zr_context* ctx) {
 }
 
 static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_tokens, uint32_t* d_out_tokens,
-                             float* d_out_logits, float* h_partials) {
+                             float* d_out_logits, float* h_partials, bool waits) {
     zr_status rc = check_ready(ctx);
     if (rc) return rc;
     const zr_model_desc& d = ctx->desc;
@@ -629,7 +629,8 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
         } else {
             if ((rc = launch_rms_norm(ctx, hidden, o, hidden, L.mlp_norm, nullptr, ctx->xa, lo, nullptr, T, H)))
                 return rc;
-            if ((rc = launch_gemm(ctx, ctx->xa, L.w_gate_up, nullptr, ctx->ffn_a, T, 2 * F, H, kEpiSwiGLU)))
+            if ((rc = launch_gemm(ctx, ctx->xa, L.w_gate_up, nullptr, ctx->ffn_a, T, 2 * F, H, kEpiSwiGLU, nullptr,
+                                  waits)))
                 return rc;
         }
         down = Slabs(ctx->proj);
@@ -981,7 +982,7 @@ zr_status zr_forward_staged_async(zr_context* ctx, zr_staged* s, const uint32_t*
                                   float* d_out_logits) {
     StagedMeta* st = (StagedMeta*)s;
     if (!ctx || !st || st->ctx != ctx) return set_global_err(ZR_E_INVALID, "staged microbatch of another context");
-    return run_forward(ctx, st, d_tokens, d_out_tokens, d_out_logits, nullptr);
+    return run_forward(ctx, st, d_tokens, d_out_tokens, d_out_logits, nullptr, false);
 }
 
 zr_status zr_synchronize(zr_context* ctx) {
@@ -1024,7 +1025,7 @@ zr_status zr_graph_capture_staged(zr_context* ctx, zr_staged* s, const uint32_t*
     ZR_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const bool pending = ctx->token_check_pending;
     ZR_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    zr_status rc = run_forward(ctx, st, d_tokens, d_out_tokens, d_out_logits, nullptr);
+    zr_status rc = run_forward(ctx, st, d_tokens, d_out_tokens, d_out_logits, nullptr, false);
     hipGraph_t graph = nullptr;
     const hipError_t e_end = hipStreamEndCapture(ctx->stream, &graph);
     ctx->token_check_pending = pending;  // nothing ran yet
@@ -1199,7 +1200,7 @@ zr_status step_graph_capture(zr_step_graph* g, int b, const uint32_t* in, uint32
     const bool pending = ctx->token_check_pending;
     ZR_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     zr_status rc = launch_pack(ctx, &g->st[b]);
-    if (!rc) rc = run_forward(ctx, &g->st[b], in, out, nullptr, nullptr);
+    if (!rc) rc = run_forward(ctx, &g->st[b], in, out, nullptr, nullptr, g == ctx->fwd_graph);
     hipGraph_t graph = nullptr;
     const hipError_t e_end = hipStreamEndCapture(ctx->stream, &graph);
     ctx->token_check_pending = pending;  // nothing ran yet
@@ -1376,7 +1377,7 @@ zr_status zr_forward(zr_context* ctx, const zr_microbatch* mb, uint32_t* out_tok
         return forward_replayed(ctx, mb, out_tokens);
     StagedMeta* st = ctx->scratch_stage;
     zr_status rc = stage_microbatch(ctx, mb, st);
-    if (!rc) rc = run_forward(ctx, st, nullptr, ctx->tokens_out, nullptr, out_partials);
+    if (!rc) rc = run_forward(ctx, st, nullptr, ctx->tokens_out, nullptr, out_partials, true);
     if (!rc && out_tokens)
         ZR_HIP(ctx, hipMemcpyAsync(out_tokens, ctx->tokens_out, 4 * (size_t)mb->num_seqs, hipMemcpyDeviceToHost,
                                    ctx->stream));
@@ -1889,7 +1890,7 @@ static zr_status run_gemm_op(zr_context* ctx, const float* d_a, uint16_t* packed
     if (e != hipSuccess) rc = set_err(ctx, ZR_E_OOM, "gemm workspace: %s", hipGetErrorString(e));
     if (!rc) rc = launch_to_bf16_pair(ctx, a_pad, m, kp, a16, lo);
     if (!rc && epilogue == kEpiSwiGLU) {
-        rc = launch_gemm(ctx, a16, packed, nullptr, h16, m, n, kp, kEpiSwiGLU);
+        rc = launch_gemm(ctx, a16, packed, nullptr, h16, m, n, kp, kEpiSwiGLU, nullptr, true);
         if (!rc) rc = launch_from_bf16_pair(ctx, h16, m, n / 2, lo, d_out);
     } else if (!rc) {
         rc = launch_gemm(ctx, a16, packed, d_out, nullptr, m, n, kp, kEpiStore);

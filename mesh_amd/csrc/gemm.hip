@@ -857,47 +857,90 @@ static GemmChoice one_pass(const GemmCfg& c, int m, int n, int k) {
     return best;
 }
 
-// Tiles of products over many rows, priced by how they fill the CUs.  A block
-// of a config takes `step` us per k-step of 32 (plus four of prologue and
-// epilogue) in a full pass over its slots; a last pass over a share f of them
-// takes alone + (1 - alone) f of that, less than a whole one because the chip
-// clocks higher then (it runs these products at its power limit: full passes
-// reach 1.34-1.44 PFLOP/s of MFMA work whatever the tile).  Fitted to cold
-// weights, hi + lo operands, 256-3000 rows, 2048-28672 columns, K 2048-14336;
-// within 5 % of most of them.  With two blocks per CU, up to half of the slots
-// run one to a CU.
+// Tiles of products over many rows, priced two ways.
+//
+// By themselves: a block of a config takes `step` us per k-step of 32 (plus
+// four of prologue and epilogue) in a full pass over its slots; a last pass
+// over a share f of them takes alone + (1 - alone) f of that, less than a whole
+// one because the chip clocks higher then (it runs these products at its power
+// limit: full passes reach 1.34-1.44 PFLOP/s of MFMA work whatever the tile).
+// Fitted to cold weights, hi + lo operands, 256-3000 rows, 2048-28672 columns,
+// K 2048-14336; within 5 % of most of them.  With two blocks per CU, up to half
+// of the slots run one to a CU.
+//
+// Beside other streams' kernels: those fill the CUs that a last pass leaves, so
+// a product costs the CU time it takes, blocks x `busy` us per k-step (plus
+// `fixed` steps) over the slots.  Three streams of one product each (the same
+// sizes) are within 3 % of it.  Per element of the product 256 x 256 tiles take
+// 0.91 and 64 x 256 ones 1.14 of the CU time of 128 x 256 tiles.
 struct TileCost {
     GemmCfg cfg;
     int per_cu;
     float step, alone;
+    struct { float busy, fixed; } store, fused;
 };
 static const TileCost kTileCosts[] = {
-    {{2, 2, 2, 4, 3}, 1, 0.80f, 0.70f},  // 128 x 256
-    {{2, 2, 3, 4, 3}, 1, 1.10f, 0.60f},  // 192 x 256, 12 waves
-    {{2, 2, 4, 4, 3}, 1, 1.47f, 0.50f},  // 256 x 256, 16 waves
-    {{2, 2, 1, 4, 3}, 2, 0.90f, 0.70f},  // 64 x 256, two blocks per CU
+    {{2, 2, 2, 4, 3}, 1, 0.80f, 0.70f, {0.883f, 2.0f}, {0.863f, 5.6f}},  // 128 x 256
+    {{2, 2, 3, 4, 3}, 1, 1.10f, 0.60f, {1.273f, 0.3f}, {1.232f, 6.7f}},  // 192 x 256, 12 waves
+    {{2, 2, 4, 4, 3}, 1, 1.47f, 0.50f, {1.628f, 0.0f}, {1.564f, 7.1f}},  // 256 x 256, 16 waves
+    {{2, 2, 1, 4, 3}, 2, 0.90f, 0.70f, {0.936f, 0.7f}, {0.986f, 0.0f}},  // 64 x 256, two blocks per CU
+    {{2, 4, 2, 4, 3}, 1, 1.55f, 0.60f, {1.620f, 6.0f}, {1.620f, 6.0f}},  // 128 x 512
 };
 
-static GemmChoice cheapest(int m, int n, int k, bool may_split) {
-    // priced at whole 64-row units, so that a plan (and its workspace) changes
-    // at their ends only
+// us per float of a split-K slab past the first: written, then read by the
+// product's consumer
+constexpr float kSlabUs = 1.6e-6f;
+
+// (both priced at whole 64-row units, so that a plan and its workspace change
+// at their ends only)
+static int tiles_of(const TileCost& t, int rows, int n) {
+    return ((rows + t.cfg.bm() - 1) / t.cfg.bm()) * ((n + t.cfg.bn() - 1) / t.cfg.bn());
+}
+
+static float time_alone(const TileCost& t, int splits, int rows, int n, int k) {
+    const int KT = (k + 31) / 32, slots = t.per_cu * device_cus();
+    const int blocks = tiles_of(t, rows, n) * splits, full = blocks / slots;
+    const float f = (float)(blocks - full * slots) / slots;
+    float passes = (float)full;
+    if (f > 0.0f) passes += t.per_cu == 2 && f <= 0.5f ? 0.45f + 0.15f * f : t.alone + (1.0f - t.alone) * f;
+    return passes * t.step * ((KT + splits - 1) / splits + 4) + kSlabUs * rows * (float)n * (splits - 1);
+}
+
+static float cu_time(const TileCost& t, int splits, int rows, int n, int k, int epilogue) {
+    const int KT = (k + 31) / 32;
+    const auto& c = epilogue == kEpiStore ? t.store : t.fused;
+    return (float)(tiles_of(t, rows, n) * splits) / (t.per_cu * device_cus()) * c.busy *
+               ((KT + splits - 1) / splits + c.fixed) +
+           kSlabUs * rows * (float)n * (splits - 1);
+}
+
+// The plan that is fastest by itself among those that take no more CU time
+// than `most` does (the plan of one pass over the CUs).  Without that limit the
+// tiles that fill a pass better are up to 6 % slower per microbatch where
+// others run beside it (4 layers on three streams, us: Llama-3, 600 rows 2352
+// against 2232 with it, 1400 rows 4722 / 4457; TinyLlama, 8 layers, 800 rows
+// 1470 / 1428), and 0-5 % faster where none do.
+// waits: no limit -- the caller waits for this microbatch, and nothing else of
+// its context runs beside it.
+static GemmChoice cheapest(int m, int n, int k, int epilogue, const GemmChoice& most, bool waits) {
     const int rows = (m + 63) / 64 * 64, KT = (k + 31) / 32, cus = device_cus();
-    GemmChoice best{kTileCosts[0].cfg, 1};
-    float least = 1e30f;
+    auto same = [](const GemmCfg& a, const GemmCfg& b) {
+        return a.wm == b.wm && a.wn == b.wn && a.waves_m == b.waves_m && a.waves_n == b.waves_n;
+    };
+    float limit = 1e30f, least = 1e30f;
+    for (const TileCost& t : kTileCosts)
+        if (same(t.cfg, most.cfg)) {
+            if (!waits) limit = cu_time(t, most.splits, rows, n, k, epilogue);
+            least = time_alone(t, most.splits, rows, n, k);
+        }
+    GemmChoice best = most;
     for (const TileCost& t : kTileCosts) {
-        const int tiles = ((rows + t.cfg.bm() - 1) / t.cfg.bm()) * ((n + t.cfg.bn() - 1) / t.cfg.bn());
-        const int slots = t.per_cu * cus;
-        for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
+        const int tiles = tiles_of(t, rows, n);
+        for (int s = 1; s <= (epilogue == kEpiStore ? 16 : 1); ++s) {
             if (s > 1 && KT / s < 4) break;
             if (s > 4 && tiles * s > 2 * cus) break;  // (bounds the workspace)
-            const int blocks = tiles * s, full = blocks / slots;
-            const float f = (float)(blocks - full * slots) / slots;
-            float passes = (float)full;
-            if (f > 0.0f)
-                passes += t.per_cu == 2 && f <= 0.5f ? 0.45f + 0.15f * f : t.alone + (1.0f - t.alone) * f;
-            // each split past the first: one more f32 slab written and read at ~5 TB/s
-            const float us = passes * t.step * ((KT + s - 1) / s + 4) + 8e-6f / 5 * rows * (float)n * (s - 1);
-            if (us < least) {
+            const float us = time_alone(t, s, rows, n, k);
+            if (us < least && cu_time(t, s, rows, n, k, epilogue) <= limit) {
                 least = us;
                 best = {t.cfg, s};
             }
@@ -909,7 +952,7 @@ static GemmChoice cheapest(int m, int n, int k, bool may_split) {
 // The tile and K split of a product (measured with weights streamed from HBM
 // and split activations; the decode steps are those of TinyLlama and Llama-3
 // shapes).
-static GemmChoice choose_tiles(int m, int n, int k, int epilogue) {
+static GemmChoice choose_tiles(int m, int n, int k, int epilogue, bool waits) {
     const bool store = epilogue == kEpiStore;
     // A vocabulary-wide head over 129-256 rows (the 256-session decode step):
     // 256 x 256 tiles in 16-wave blocks, four waves per SIMD (128256 columns:
@@ -920,13 +963,23 @@ static GemmChoice choose_tiles(int m, int n, int k, int epilogue) {
         // fill twice the CUs of one 128-row block (decode steps at 96 / 128
         // sessions -4.7 / -4.2 %)
         if (m <= 128) return {{2, 2, 1, 4, 3}, 1};
-        const GemmChoice c = cheapest(m, n, k, false);
         // 129-256 rows: 128 x 256 tiles in 16-wave blocks (32 x 64 wave tiles,
         // four waves per SIMD to cover the copies' latency): GEMM class
         // 7.33-7.36 against 7.47-7.50 ms per 256-session step with 8 waves.
-        // The store products measured slower in 16-wave blocks.
-        if (m <= 256 && c.cfg.bm() == 128) return {{1, 2, 4, 4, 3}, 1};
-        return c;
+        // The store products measured slower in 16-wave blocks.  64 x 256 tiles
+        // are faster by themselves where 128-row ones leave CUs idle (256 rows,
+        // 11264 columns, K 2048: 35 / 45 us) and slower beside other streams
+        // (steps of 208 sessions on three streams, 8 TinyLlama layers: 778 / 751
+        // us; 4 layers of a Llama-3 shard: 1037 / 1011).
+        if (m <= 256) {
+            const GemmChoice w16 = {{1, 2, 4, 4, 3}, 1};
+            if (!waits) return w16;
+            const GemmChoice c = cheapest(m, n, k, epilogue, {{2, 2, 2, 4, 3}, 1}, true);
+            return c.cfg.bm() == 128 && c.cfg.bn() == 256 ? w16 : c;
+        }
+        // 128 x 512 tiles once they alone fill two passes over the CUs
+        const bool wide = ((m + 127) / 128) * ((n + 511) / 512) >= 2 * device_cus();
+        return cheapest(m, n, k, epilogue, {wide ? GemmCfg{2, 4, 2, 4, 3} : GemmCfg{2, 2, 2, 4, 3}, 1}, waits);
     }
     // <= 32 rows: a 4-deep ring and one pass of splits over the CUs (TinyLlama
     // shapes at 32 rows, back to back with weights from HBM: QKV 4.84 us
@@ -946,16 +999,18 @@ static GemmChoice choose_tiles(int m, int n, int k, int epilogue) {
     if (m <= 128 && store && n < 65536) return one_pass({2, 1, 1, 4, 4}, m, n, k);
     // vocabulary-wide heads: 256-row tiles read each weight tile once
     if (n >= 65536) return one_pass(m > 128 ? GemmCfg{2, 4, 4, 2, 3} : GemmCfg{2, 4, 2, 4, 3}, m, n, k);
-    if (m <= 256) return one_pass(n >= 16384 ? GemmCfg{2, 4, 2, 4, 3} : GemmCfg{2, 2, 2, 4, 3}, m, n, k);
-    // More rows (us per product, the rules before -- 128 x 256 tiles, up to 4
-    // splits past one pass -- against these): Llama-3 at 2108 rows QKV 198 /
-    // 186, O 143 / 135 and no slabs, down 436 / 424 (no slabs), at 997 gate/up
-    // 401 / 374, at 520 288 / 232; TinyLlama at 997 gate/up 104 / 89, at 2108
-    // QKV 90 / 50, down 118 / 93.
-    return cheapest(m, n, k, true);
+    const GemmChoice plain = one_pass(n >= 16384 ? GemmCfg{2, 4, 2, 4, 3} : GemmCfg{2, 2, 2, 4, 3}, m, n, k);
+    if (m <= 256) return plain;
+    // More rows (us per product by itself / beside two more streams, one pass of
+    // 128 x 256 tiles and up to 4 splits against this): Llama-3 at 2108 rows QKV
+    // 202 / 186 against 187 / 179, O 150 / 129 against 137 / 115 and no slabs,
+    // down 479 / 456 against 405 / 432, gate/up at 1000 408 / 394 against 380 /
+    // 366; TinyLlama at 1000 gate/up 103 / 82 against 88 / 76, at 300 QKV 12.9 /
+    // 11.5 against 12.4 / 8.6 with half the slabs.
+    return cheapest(m, n, k, epilogue, plain, false);
 }
 
-GemmPlan gemm_plan(int m, int n, int k, int epilogue) {
+GemmPlan gemm_plan(int m, int n, int k, int epilogue, bool waits) {
     GemmPlan p;
     if (few_rows(m, n, epilogue)) {
         p.few_rows = true;
@@ -978,7 +1033,7 @@ GemmPlan gemm_plan(int m, int n, int k, int epilogue) {
         p.kt_per_split = p.KT;
         return p;  // one launch, no workspace
     }
-    const GemmChoice ch = choose_tiles(m, n, k, epilogue);
+    const GemmChoice ch = choose_tiles(m, n, k, epilogue, waits);
     const GemmCfg& c = ch.cfg;
     p.wm = c.wm;
     p.wn = c.wn;
@@ -1065,7 +1120,7 @@ zr_status launch_norm_gemm(zr_context* ctx, const float* x, const Slabs& residua
 }
 
 zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_packed, float* c_f32,
-                      uint16_t* c_bf16, int m, int n, int k, int epilogue, Slabs* deferred) {
+                      uint16_t* c_bf16, int m, int n, int k, int epilogue, Slabs* deferred, bool waits) {
     if (deferred && (epilogue != kEpiStore || !c_f32 || c_bf16))
         return set_err(ctx, ZR_E_INVARIANT, "deferred split-K needs an f32 store epilogue");
     if (m <= 0) return ZR_OK;
@@ -1075,7 +1130,7 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
     if (a_bytes > 0x7fffffffull || w_bytes > 0x7fffffffull)
         return set_err(ctx, ZR_E_UNSUPPORTED, "GEMM operands of %zu / %zu bytes exceed 2 GiB", a_bytes, w_bytes);
     const bool split_act = (ctx->desc.flags & ZR_FLAG_SPLIT_ACTIVATIONS) != 0;
-    const GemmPlan p = gemm_plan(m, n, k, epilogue);
+    const GemmPlan p = gemm_plan(m, n, k, epilogue, waits);
     const bool in_launch = p.few_rows ? epilogue == kEpiSwiGLU : swiglu_ksplit(m, n, k, epilogue);
     if (in_launch && (!c_bf16 || c_f32 || deferred))
         return set_err(ctx, ZR_E_INVARIANT, "K-split SwiGLU (M=%d) writes the bf16 operand only", m);
@@ -1137,6 +1192,7 @@ zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_pack
             gemm_launch<WMV, WNV, WAM, WAN, ST, 1, 1>(p, ctx->stream, a, m, k, w_packed, nullptr, n, 0, c_bf16, 0); \
         launched = true;                                                                               \
     }
+    ZR_GEMM_FUSED_CASE(2, 4, 2, 4, 3)
     ZR_GEMM_FUSED_CASE(2, 2, 2, 4, 3)
     ZR_GEMM_FUSED_CASE(2, 2, 1, 4, 3)
     ZR_GEMM_FUSED_CASE(1, 2, 4, 4, 3)

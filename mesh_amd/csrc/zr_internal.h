@@ -437,14 +437,16 @@ struct GemmPlan {
     bool direct = true;
     size_t ws_floats = 0;
 };
-GemmPlan gemm_plan(int m, int n, int k, int epilogue);
+// waits: the caller waits for the microbatch; the tiles of a fused gate / up
+// product (not its bits) then follow its time by itself, otherwise its CU time.
+GemmPlan gemm_plan(int m, int n, int k, int epilogue, bool waits = false);
 // C = A @ W (W packed, A bf16 operand).  kEpiStore writes c_f32; kEpiSwiGLU
 // writes silu(gate) * up as the bf16 operand c_bf16 (or f32 c_f32).  With
 // `deferred` (kEpiStore only) a split-K product is left as its slabs in the
 // split-K workspace for the consumer to sum (valid until the next GEMM);
 // *deferred then describes C either way.
 zr_status launch_gemm(zr_context* ctx, const uint16_t* a, const uint16_t* w_packed, float* c_f32,
-                      uint16_t* c_bf16, int m, int n, int k, int epilogue, Slabs* deferred = nullptr);
+                      uint16_t* c_bf16, int m, int n, int k, int epilogue, Slabs* deferred = nullptr, bool waits = false);
 constexpr int kNormRows = 2, kNormCols = 4096;  // the most rows / columns normalised inside a product
 // The product of rms_norm(x + residual) gamma in one launch, for the few rows
 // norm_in_gemm takes (its plan has no split-K slabs: the residual's may lie in

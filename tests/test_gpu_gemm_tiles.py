@@ -7,10 +7,14 @@ leaving a form without a test.
 """
 import ctypes as C
 
+import numpy as np
 import pytest
 
-from mesh_amd import _lib
+from mesh_amd import BackendMicrobatchExecutor, DeviceBuffer, _lib
 from tests import test_gpu_kernels as kernels
+from tests.gpu_util import stage_mixed
+from tests.test_gpu_model import make
+from tests.testmodels import geometry, random_weights
 
 STORE, SWIGLU = 0, 1
 
@@ -22,10 +26,15 @@ class GemmPlan(C.Structure):
                [("direct", C.c_bool), ("ws_floats", C.c_size_t)]
 
 
-def gemm_plan(m, n, k, epilogue):
-    fn = C.CDLL(_lib.LIB_PATH)._ZN2zr9gemm_planEiiii
-    fn.restype, fn.argtypes = GemmPlan, [C.c_int] * 4
-    return fn(m, n, k, epilogue)
+def gemm_plan(m, n, k, epilogue, waits=True):
+    """waits: of a call that waits for its microbatch, as the op entries and zr_forward do."""
+    fn = C.CDLL(_lib.LIB_PATH)._ZN2zr9gemm_planEiiiib
+    fn.restype, fn.argtypes = GemmPlan, [C.c_int] * 4 + [C.c_bool]
+    return fn(m, n, k, epilogue, waits)
+
+
+def tile(p):
+    return p.wm * p.waves_m * 32, p.wn * p.waves_n * 32
 
 
 # (m, k, f, k-steps per wave of 4)
@@ -56,7 +65,7 @@ REDUCED = [(9, 64, 32, 32, 1), (11, 96, 96, 32, 1), (23, 320, 320, 32, 2), (32, 
 @pytest.mark.parametrize("m,k,f,bm,splits", REDUCED)
 def test_reduced_cases_take_the_tiles_they_name(m, k, f, bm, splits):
     p = gemm_plan(m, 2 * f, k, SWIGLU)
-    assert (p.few_rows, p.wm * p.waves_m * 32, p.wn * p.waves_n * 32, p.splits, p.direct) == (False, bm, 128, splits, False)
+    assert (p.few_rows, tile(p), p.splits, p.direct) == (False, (bm, 128), splits, False)
 
 
 @pytest.mark.gpu
@@ -64,3 +73,99 @@ def test_reduced_cases_take_the_tiles_they_name(m, k, f, bm, splits):
 @pytest.mark.parametrize("m,k,f,bm,splits", REDUCED)
 def test_swiglu_in_the_slab_reduce(split, m, k, f, bm, splits):
     kernels.test_gemm_swiglu_matches_fp64(split, m, k, f)
+
+
+# Past 64 rows: (m, k, f, tile, column blocks left over by the 8 XCDs)
+FUSED = [(100, 256, 512, (64, 256), 4),
+         (130, 200, 96, (64, 256), 1),
+         (700, 320, 2080, (64, 256), 1),     # 11 row blocks
+         (1009, 320, 2848, (128, 256), 7),   # 8 waves of 64 x 64
+         (401, 1024, 5664, (128, 256), 5),
+         (777, 256, 10272, (192, 256), 1),
+         (1009, 320, 5664, (256, 256), 5),
+         (997, 2048, 5632, (256, 256), 4),   # a 997-row TinyLlama prompt's gate / up
+         (600, 64, 50016, (128, 512), 4),
+         (1100, 320, 14336, (128, 512), 0)]
+
+
+@pytest.mark.parametrize("m,k,f,shape,left", FUSED)
+def test_fused_cases_take_the_tiles_they_name(m, k, f, shape, left):
+    p = gemm_plan(m, 2 * f, k, SWIGLU)
+    assert (tile(p), p.splits, p.direct, p.col_blocks % 8) == (shape, 1, True, left)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("m,k,f,shape,left", FUSED)
+def test_fused_swiglu_tiles(split, m, k, f, shape, left):
+    """Rows and columns that end inside a tile; (column block, split) pairs
+    left over by the 8 XCDs, whose row blocks go round all of them."""
+    kernels.test_gemm_swiglu_matches_fp64(split, m, k, f)
+
+
+# (m, k, n, tile, splits, pairs left over by 8)
+STORED = [(300, 128, 64, (64, 256), 1, 1),
+          (700, 512, 4100, (64, 256), 1, 1),
+          (389, 4096, 1000, (64, 256), 8, 0),
+          (300, 4096, 1024, (64, 256), 10, 0),    # the last split shorter
+          (260, 4096, 512, (64, 256), 13, 2),
+          (261, 8192, 250, (64, 256), 16, 0),
+          (997, 2048, 2560, (128, 256), 3, 6),    # a 997-row TinyLlama prompt's QKV
+          (1009, 2048, 2500, (128, 256), 3, 6),
+          (2100, 512, 2050, (128, 256), 1, 1),
+          (1200, 1000, 8100, (192, 256), 1, 0),
+          (1009, 320, 11300, (256, 256), 1, 5),
+          (600, 256, 20000, (128, 512), 1, 0)]
+
+
+@pytest.mark.parametrize("m,k,n,shape,splits,left", STORED)
+def test_stored_cases_take_the_tiles_they_name(m, k, n, shape, splits, left):
+    for waits in (True, False):
+        p = gemm_plan(m, n, k, STORE, waits)
+        assert (tile(p), p.splits, p.col_blocks * p.splits % 8) == (shape, splits, left)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("m,k,n,shape,splits,left", STORED)
+def test_store_tiles(split, m, k, n, shape, splits, left):
+    kernels.test_gemm_matches_fp64(split, m, k, n)
+
+
+# Microbatches beside other streams: gate / up takes no more CU time than 128 x
+# 256 tiles (128 x 512 ones that fill two passes), whatever fills a pass better.
+# (rows, k, f, tile of a waiting call, of an asynchronous one)
+BESIDE = [(200, 2048, 5632, (64, 256), (128, 256)), (256, 4096, 7168, (64, 256), (128, 256)),
+          (600, 4096, 14336, (192, 256), (128, 256)), (640, 4096, 7168, (192, 256), (128, 512)),
+          (1400, 4096, 14336, (128, 256), (128, 512)), (997, 2048, 5632, (256, 256), (256, 256))]
+
+
+@pytest.mark.parametrize("m,k,f,alone,beside", BESIDE)
+def test_asynchronous_microbatches_take_tiles_by_their_cu_time(m, k, f, alone, beside):
+    plans = [gemm_plan(m, 2 * f, k, SWIGLU, w) for w in (True, False)]
+    assert [tile(p) for p in plans] == [alone, beside]
+    work = {(128, 256): 0.863, (192, 256): 1.232, (256, 256): 1.564, (64, 256): 0.493, (128, 512): 1.62}
+    blocks = -(-m // 128) * (-(-2 * f // 256))
+    assert plans[1].row_blocks * plans[1].col_blocks * work[beside] <= 1.03 * blocks * work[128, 256]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [200, 700, 1000])
+def test_waiting_and_asynchronous_calls_agree_bit_for_bit(rows):
+    """The tiles differ, the sums do not: one chunk through zr_forward and
+    through zr_forward_staged_async."""
+    cfg = dict(hidden=256, num_heads=4, num_kv_heads=2, num_layers=2, vocab=300, ffn=7168, rms_norm_eps=1e-5,
+               rope_base=10000.0)
+    assert len({tile(gemm_plan(rows, 2 * cfg["ffn"], cfg["hidden"], SWIGLU, w)) for w in (True, False)}) == 2
+    geo = geometry(cfg)
+    ctx, _ = make(cfg, geo, random_weights(cfg, geo, seed=5), "bf16", True, max_tokens=1000, max_seqs=2, pages=256,
+                  pps=80)
+    toks = np.random.default_rng(rows).integers(0, cfg["vocab"], rows).astype(np.uint32)
+    _, want = BackendMicrobatchExecutor.forward_mixed([ctx.new_backend(2048)], [toks.tolist()])
+    st = stage_mixed(ctx, [ctx.new_backend(2048)], [rows], toks)
+    d_ids, d_logits = DeviceBuffer(ctx, 4), DeviceBuffer(ctx, 4 * cfg["vocab"])
+    ctx.check(ctx.lib.zr_forward_staged_async(ctx.h, st, None, d_ids.ptr, d_logits.ptr))
+    ctx.check(ctx.lib.zr_synchronize(ctx.h))
+    np.testing.assert_array_equal(d_logits.download(np.float32, (1, cfg["vocab"])), want)
+    ctx.lib.zr_staged_destroy(st)
+    ctx.close()

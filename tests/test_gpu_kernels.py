@@ -725,7 +725,7 @@ def test_kv_gather_scatter_round_trip_with_partial_first_page(kv_dtype):
 @pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("m,k,n", [(1, 64, 100), (7, 256, 4112), (32, 2048, 2048), (100, 512, 1000),
                                    (256, 4096, 1024), (300, 128, 64), (128, 4104, 4112), (130, 520, 66000),
-                                   # more 128 x 256 tiles than CUs: K split 3 and 4 ways to fill the last pass
+                                   # 192 x 256 tiles, unsplit and split 4 ways
                                    (2108, 4096, 4096), (2108, 14336, 4096),
                                    # the 256-row decode products (QKV, O, down) and a head over
                                    # 16-wave 256 x 256 tiles
@@ -764,9 +764,9 @@ def test_gemm_matches_fp64(split, m, k, n):
                                    (32, 2048, 5632),     # the 32-session TinyLlama gate / up: K over 4 waves
                                    (1, 128, 64), (7, 256, 96), (5, 96, 64),  # at most 8 rows: weights to registers
                                    (100, 256, 512),      # 65-128 rows: fused, 64 x 256 tiles
-                                   (130, 200, 96),       # fused, 128 x 256 tiles, K padded to 224
+                                   (130, 200, 96),       # fused, 64 x 256 tiles, K padded to 224
                                    (256, 4096, 14336),   # the Llama-3-8B gate / up product of the decode step
-                                   (2108, 1024, 2048)])  # prefill-sized: fused 128 x 512 tiles
+                                   (2108, 1024, 2048)])  # prefill-sized: fused, 192 x 256 tiles
 def test_gemm_swiglu_matches_fp64(split, m, k, f):
     # h = silu(A @ Wg) * (A @ Wu) (tensor_ops.rs:268-278, forward_pass.rs:2286-2289)
     geo = ModelGeometry(hidden=256, num_heads=4, num_kv_heads=4, num_layers=1, vocab=64, ffn=256)

@@ -222,9 +222,8 @@ def test_mixed_chunked_prefill_and_decode_microbatch():
 
 
 def test_prefill_rows_wide_ffn_partials():
-    """1200 prefill rows against FFN 14336: the gate/up GEMM takes its
-    128 x 512-column fused SwiGLU tiles (10 x 56 tiles, two passes over the
-    CUs).  Per-layer pre-all-reduce partials (O, down) and logits against the
+    """1200 prefill rows against FFN 14336: the gate/up GEMM takes 256 x 256
+    fused SwiGLU tiles (5 x 112, more than two passes over the CUs).  Per-layer pre-all-reduce partials (O, down) and logits against the
     oracle; the second chunk continues a page-unaligned 300-row prefix."""
     cfg = dict(hidden=256, num_heads=4, num_kv_heads=2, num_layers=1, vocab=512, ffn=14336, rms_norm_eps=1e-5,
                rope_base=10000.0)
