@@ -249,7 +249,8 @@ zr_status zr_attention(zr_context* ctx, zr_staged* st, int layer, const float* d
  * 16-byte nontemporal page loads in the same order, without Q, softmax, MFMA
  * or output -- and returns the mean launch time in *mean_ms (HIP events on
  * the context stream; synchronises).  Needs the MFMA page layout (head_dim 64
- * or 128) and decode attention items in `st`.  For a bench or a profiler:
+ * or 128) and decode attention items in `st`, or prompt chunks in an f32 pool
+ * (alone, their rows are probed as decode tiles).  For a bench or a profiler:
  * dividing the launch's K/V bytes by it gives the ceiling that the attention
  * kernel's own rate is measured against. */
 zr_status zr_kv_read_probe(zr_context* ctx, zr_staged* st, int layer, int repeats, double* mean_ms);

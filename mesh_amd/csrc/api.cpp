@@ -192,6 +192,27 @@ void stage_fixed_bytes(const zr_context* ctx, int S, int total_q, const StageFix
     *dev_bytes = b.total_bytes;
 }
 
+// Pages per split of the decode kernel's tiles: ~96 at 256 sessions x 8 kv
+// heads x ~1.5k tokens (measured best on MI355X with longest-first dispatch:
+// 64 and 144 tie); at least 8, which measured best at 32 sessions (a launch
+// there costs ~8 us plus ~0.45 us per page of a split: 12 pages 0.4 % slower,
+// 16 1.2 %, 24 6 %); and at most 16 splits per tile, which the merge combines in
+// one round trip; more take its general form (32 sessions at 3.5-4k contexts:
+// 1.98 ms per step with 8-page splits, 32 per tile, against 1.76-1.81 with 16).
+static int pages_per_split(const std::vector<int>& tile_pages, int kv_heads) {
+    const long target_wgs = 2048;
+    long total = 0;
+    int longest = 0;
+    for (int p : tile_pages) {
+        total += p;
+        longest = std::max(longest, p);
+    }
+    int pps = (int)std::min<long>(4096, std::max<long>(8, (total * kv_heads + target_wgs - 1) / target_wgs));
+    pps = std::max(pps, (longest + 15) / 16);
+    if (const char* env = getenv("ZR_ATTN_PAGES_PER_SPLIT")) pps = std::max(1, atoi(env));
+    return pps;
+}
+
 zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta* st, const StageFixed* fixed,
                            bool* fits) {
     if (fits) *fits = true;
@@ -285,7 +306,7 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     }
     std::vector<int> tile_pages;
     std::vector<int4> pblk;  // prefill blocks {seq, r0, nrows, pages}
-    long total_pages = 0, total_ktiles = 0;
+    long total_ktiles = 0;
     for (int s = 0; s < S && qpt > 0; ++s) {
         const int ql = mb->q_len[s], kb = mb->kv_before[s], fo = mb->first_offset[s];
         if (prows && ql >= prows && (!f32_kv || (long)ql * G * (kb + ql / 2) >= kPrefillF32Work)) {
@@ -304,24 +325,9 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
             const int pages = (fo + last_visible + 1 + kPageRows - 1) / kPageRows;
             st->h_tiles.push_back(make_int4(s, q0, nq, 0));
             tile_pages.push_back(pages);
-            total_pages += pages;
         }
     }
-    // ~96 pages per split at 256 sessions x 8 kv heads x ~1.5k tokens (measured
-    // best on MI355X with longest-first dispatch: 64 and 144 tie); at least 8
-    // pages, which measured best at 32 sessions (a launch there costs ~8 us
-    // plus ~0.45 us per page of a split: 12 pages 0.4 % slower, 16 1.2 %, 24 6 %)
-    const long target_wgs = 2048;
-    int pps = (int)std::min<long>(4096, std::max<long>(8, (total_pages * ctx->local_kv_heads + target_wgs - 1) / target_wgs));
-    // and at most 16 splits per tile, which the merge combines in one round
-    // trip; more take its general form (32 sessions at 3.5-4k contexts: 1.98
-    // ms per step with 8-page splits, 32 per tile, against 1.76-1.81 with 16)
-    {
-        int max_pages = 0;
-        for (int tp : tile_pages) max_pages = std::max(max_pages, tp);
-        pps = std::max(pps, (max_pages + 15) / 16);
-    }
-    if (const char* env = getenv("ZR_ATTN_PAGES_PER_SPLIT")) pps = std::max(1, atoi(env));
+    const int pps = pages_per_split(tile_pages, ctx->local_kv_heads);
     for (size_t t = 0; t < st->h_tiles.size(); ++t) {
         st->h_tiles[t].w = (int)st->h_items.size();
         for (int pb = 0; pb < tile_pages[t]; pb += pps)
@@ -1445,6 +1451,38 @@ zr_status zr_attention(zr_context* ctx, zr_staged* s, int layer, const float* d_
     return rc;
 }
 
+static std::vector<int4> decode_records(zr_context* ctx, const StagedMeta* st) {
+    const BlobLayout L = blob_layout(st->num_seqs, st->stride, st->total_q, st->grid_items, st->grid_merge,
+                                     st->n_pblocks, ctx->head_dim);
+    const int* first_offset = (const int*)(st->h_blob.data() + L.o_foff);
+    const int* tables = (const int*)(st->h_blob.data() + L.o_bt);
+    const int qpt = 16 / ctx->q_per_kv;
+    std::vector<int4> tiles;  // {seq, row of the microbatch, rows, keys before the first row}
+    std::vector<int> tile_pages;
+    for (int s = 0, row = 0; s < st->num_seqs; row += st->h_q_len[s++])
+        for (int q0 = 0; q0 < st->h_q_len[s]; q0 += qpt) {
+            const int nq = std::min(qpt, st->h_q_len[s] - q0);
+            tiles.push_back(make_int4(s, row + q0, nq, st->h_kv_before[s] + q0));
+            tile_pages.push_back((first_offset[s] + st->h_kv_before[s] + q0 + nq + kPageRows - 1) / kPageRows);
+        }
+    const int pps = pages_per_split(tile_pages, ctx->local_kv_heads);
+    std::vector<int4> items;  // {tile, first page, end page}
+    for (int t = 0; t < (int)tiles.size(); ++t)
+        for (int pb = 0; pb < tile_pages[t]; pb += pps)
+            items.push_back(make_int4(t, pb, std::min(tile_pages[t], pb + pps), 0));
+    std::stable_sort(items.begin(), items.end(), [](const int4& x, const int4& y) { return x.z - x.y > y.z - y.y; });
+    std::vector<int4> rec;
+    for (const int4& it : items) {
+        const int4 t = tiles[it.x];
+        const int* bt = tables + (size_t)t.x * st->stride;
+        auto page = [&](int k) { return it.y + k < it.z ? bt[it.y + k] : 0; };
+        rec.push_back(make_int4(t.x, t.y, t.z, it.y));
+        rec.push_back(make_int4(it.z, t.w, first_offset[t.x], 0));
+        rec.push_back(make_int4(page(0), page(1), page(2), page(3)));
+    }
+    return rec;
+}
+
 zr_status zr_kv_read_probe(zr_context* ctx, zr_staged* s, int layer, int repeats, double* mean_ms) {
     StagedMeta* st = (StagedMeta*)s;
     if (!ctx || !st || !mean_ms) return set_global_err(ZR_E_INVALID, "null argument");
@@ -1452,7 +1490,14 @@ zr_status zr_kv_read_probe(zr_context* ctx, zr_staged* s, int layer, int repeats
     if (layer < 0 || layer >= ctx->desc.num_layers) return set_err(ctx, ZR_E_INVALID, "Invalid layer index: %d", layer);
     if (repeats <= 0 || repeats > 10000) return set_err(ctx, ZR_E_INVALID, "repeats %d outside 1..10000", repeats);
     if (!ctx->kv_pool) return set_err(ctx, ZR_E_INVALID, "KV pool not created");
-    return launch_kv_read_probe(ctx, st, layer, repeats, mean_ms);
+    // A microbatch of prompt chunks alone has no decode items where the chunks
+    // run as prefill blocks.  From an f32 pool that depends on the work they
+    // have, so there the probe reads the page stream of the same rows as
+    // decode tiles, which is what lighter chunks run as.
+    std::vector<int4> rec;
+    if (st->grid_items == 0 && st->n_pblocks > 0 && !ctx->plain_kv && ctx->desc.kv_dtype == ZR_DTYPE_F32)
+        rec = decode_records(ctx, st);
+    return launch_kv_read_probe(ctx, st, layer, repeats, rec, mean_ms);
 }
 
 // the page window of a gather / scatter lies inside the table and the pool

@@ -1647,20 +1647,22 @@ __global__ __launch_bounds__(64) void kv_read_probe_kernel(AttnArgs a, unsigned*
     if (lane == 0) out[blockIdx.x] = acc;
 }
 
+static size_t probe_words(const zr_context* ctx, int n_items) {
+    return (size_t)((n_items + 7) / 8) * 8 * ctx->local_kv_heads;
+}
+
 template <typename KV, int D>
-static zr_status launch_kv_read_probe_t(zr_context* ctx, StagedMeta* st, int layer, int repeats, double* mean_ms) {
+static zr_status launch_kv_read_probe_t(zr_context* ctx, StagedMeta* st, int layer, int repeats, const int4* rec,
+                                        int n_items, unsigned* words, double* mean_ms) {
     AttnArgs a{};
     a.page_elems = (size_t)2 * ctx->kv_cols * kPageRows;
     a.pool = (const KV*)ctx->kv_pool + (size_t)layer * ctx->n_pages * a.page_elems;
     a.block_tables = st->block_tables;
     a.stride = st->stride;
-    a.rec = st->attn_rec;
-    a.n_items = st->grid_items;
+    a.rec = rec;
+    a.n_items = n_items;
     a.kv_heads = ctx->local_kv_heads;
-    const dim3 grid(((st->grid_items + 7) / 8) * 8 * ctx->local_kv_heads);
-    // one word per workgroup, in the attention partials' workspace
-    if ((size_t)grid.x > ctx->attn_part_floats)
-        return set_err(ctx, ZR_E_OOM, "attention partial workspace too small for %u probe words", grid.x);
+    const dim3 grid(probe_words(ctx, n_items));
     hipEvent_t e0, e1;
     ZR_HIP(ctx, hipEventCreate(&e0));
     hipError_t e = hipEventCreate(&e1);
@@ -1671,7 +1673,7 @@ static zr_status launch_kv_read_probe_t(zr_context* ctx, StagedMeta* st, int lay
     e = hipEventRecord(e0, ctx->stream);
     for (int i = 0; i < repeats && e == hipSuccess; ++i) {
         hipLaunchKernelGGL((kv_read_probe_kernel<KV, D, sizeof(KV) == 4 ? 4 : 6>), grid, dim3(64), 0, ctx->stream, a,
-                           (unsigned*)ctx->attn_part);
+                           words);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
@@ -1685,16 +1687,41 @@ static zr_status launch_kv_read_probe_t(zr_context* ctx, StagedMeta* st, int lay
     return ZR_OK;
 }
 
-zr_status launch_kv_read_probe(zr_context* ctx, StagedMeta* st, int layer, int repeats, double* mean_ms) {
+zr_status launch_kv_read_probe(zr_context* ctx, StagedMeta* st, int layer, int repeats, const std::vector<int4>& rec,
+                               double* mean_ms) {
     if (ctx->plain_kv || (ctx->head_dim != 64 && ctx->head_dim != 128))
         return set_err(ctx, ZR_E_UNSUPPORTED, "the KV read probe follows the MFMA page layout (head_dim 64 or 128)");
-    if (st->grid_items == 0) return set_err(ctx, ZR_E_INVALID, "the staged microbatch has no decode attention items");
+    const int n_items = rec.empty() ? st->grid_items : (int)(rec.size() / 3);
+    if (n_items == 0) return set_err(ctx, ZR_E_INVALID, "the staged microbatch has no decode attention items");
+    // one word per workgroup: in the attention partials' workspace, or behind the caller's records
+    const int4* d_rec = st->attn_rec;
+    unsigned* words = (unsigned*)ctx->attn_part;
+    void* own = nullptr;
+    if (rec.empty()) {
+        if (probe_words(ctx, n_items) > ctx->attn_part_floats)
+            return set_err(ctx, ZR_E_OOM, "attention partial workspace too small for %zu probe words",
+                           probe_words(ctx, n_items));
+    } else {
+        const size_t bytes = rec.size() * sizeof(int4);
+        ZR_HIP(ctx, hipMalloc(&own, bytes + 4 * probe_words(ctx, n_items)));
+        const hipError_t e = hipMemcpy(own, rec.data(), bytes, hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(own);
+            return set_err(ctx, ZR_E_HIP, "KV read probe: %s", hipGetErrorString(e));
+        }
+        d_rec = (const int4*)own;
+        words = (unsigned*)((char*)own + bytes);
+    }
     const bool bf = ctx->desc.kv_dtype == ZR_DTYPE_BF16;
-    if (ctx->head_dim == 64)
-        return bf ? launch_kv_read_probe_t<uint16_t, 64>(ctx, st, layer, repeats, mean_ms)
-                  : launch_kv_read_probe_t<float, 64>(ctx, st, layer, repeats, mean_ms);
-    return bf ? launch_kv_read_probe_t<uint16_t, 128>(ctx, st, layer, repeats, mean_ms)
-              : launch_kv_read_probe_t<float, 128>(ctx, st, layer, repeats, mean_ms);
+    auto launch = ctx->head_dim == 64
+                      ? (bf ? launch_kv_read_probe_t<uint16_t, 64> : launch_kv_read_probe_t<float, 64>)
+                      : (bf ? launch_kv_read_probe_t<uint16_t, 128> : launch_kv_read_probe_t<float, 128>);
+    const zr_status rc = launch(ctx, st, layer, repeats, d_rec, n_items, words, mean_ms);
+    if (own) {
+        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipFree(own);
+    }
+    return rc;
 }
 
 zr_status launch_attention(zr_context* ctx, StagedMeta* st, int layer, const float* q, float* out,

@@ -407,11 +407,13 @@ zr_status launch_attention(zr_context* ctx, StagedMeta* st, int layer, const flo
 // Plain-layout pools with head_dim a multiple of 4 (tiles staged in pblocks).
 zr_status launch_attention_plain(zr_context* ctx, StagedMeta* st, int layer, const float* q, float* out_f32,
                                  uint16_t* out_bf16);
+// Times `repeats` launches of a read-only copy of the decode attention
+// launch's page stream for staged microbatch `st` at `layer` (mean ms); `rec`:
+// the records of that stream instead of the staged ones, where not empty.
+zr_status launch_kv_read_probe(zr_context* ctx, StagedMeta* st, int layer, int repeats, const std::vector<int4>& rec,
+                               double* mean_ms);
 // Pure decode microbatches (st->pure_decode): RoPE + KV append and attention in
 // one launch, q and the new K / V rows read from the QKV product's slabs.
-// Times `repeats` launches of a read-only copy of the decode attention
-// launch's page stream for staged microbatch `st` at `layer` (mean ms).
-zr_status launch_kv_read_probe(zr_context* ctx, StagedMeta* st, int layer, int repeats, double* mean_ms);
 zr_status launch_attention_rope(zr_context* ctx, StagedMeta* st, int layer, const Slabs& qkv, int rope,
                                 float* out_f32, uint16_t* out_bf16);
 zr_status launch_kv_copy(zr_context* ctx, int layer_begin, int layer_end, const int* d_table,

@@ -6,10 +6,13 @@ most 2^-17 of its value, and the lo x lo products (2^-17 again) are left out; a
 score of D products of N(0, 1) values then moves by about 2^-16 / sqrt(d) times
 sqrt(D), i.e. ~2e-5, and the weighted sum as much: 1e-4 of a row's largest
 value leaves a factor of three."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from mesh_amd import KVCacheSnapshot
+from mesh_amd import DeviceContext, KVCacheSnapshot, ModelGeometry, _lib
+from tests.gpu_util import stage_mixed
 from tests.test_gpu_attention_plain import reference, run_attention
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +70,32 @@ def test_rows_a_query_does_not_see_never_reach_it(monkeypatch, heads, kv_heads, 
     assert fine[:31].all() and not fine[31:].all()
     np.testing.assert_array_equal(np.isfinite(out)[:70], fine)
     np.testing.assert_allclose(out[:70][fine], want[:70][fine], rtol=0, atol=RTOL * np.abs(want[:70][fine]).max())
+
+
+@pytest.mark.parametrize("heads,kv_heads,D", [(32, 4, 64), (16, 8, 128)])
+def test_read_probe_of_prompt_chunks_alone(heads, kv_heads, D):
+    """zr_kv_read_probe takes a microbatch of chunks alone from an f32 pool,
+    whether they have the work for prefill blocks (600 rows on 1500) or stay on
+    decode tiles (20 rows), and leaves the pages as they were; from a bf16 pool
+    such a microbatch has no decode items."""
+    for kv_dtype, chunks, status in (("f32", [600, 601], _lib.ZR_OK), ("f32", [20], _lib.ZR_OK),
+                                     ("bf16", [600, 601], _lib.ZR_E_INVALID)):
+        geo = ModelGeometry(hidden=heads * D, num_heads=heads, num_kv_heads=kv_heads, num_layers=1, vocab=32, ffn=32)
+        ctx = DeviceContext(geo, kv_dtype=kv_dtype, max_tokens=1201, max_seqs=2, max_pages_per_seq=200)
+        ctx.create_kv_pool(300)
+        x = np.random.default_rng(D).standard_normal((1, 1500, kv_heads * D), dtype=np.float32)
+        backends = [ctx.new_backend() for _ in chunks]
+        for b in backends:
+            b.import_kv_cache(KVCacheSnapshot(1500, 1500, x, -x))
+        st = stage_mixed(ctx, backends, chunks)
+        before = [b.export_kv_cache() for b in backends]
+        ms = C.c_double()
+        assert ctx.lib.zr_kv_read_probe(ctx.h, st, 0, 5, C.byref(ms)) == status
+        if status == _lib.ZR_OK:
+            assert 0.0 < ms.value < 100.0
+        ctx.lib.zr_staged_destroy(st)
+        for b, snap in zip(backends, before):
+            after = b.export_kv_cache()
+            np.testing.assert_array_equal(after.keys, snap.keys)
+            np.testing.assert_array_equal(after.values, snap.values)
+        ctx.close()
