@@ -2,23 +2,50 @@
 
 The same sessions in a step of nine rows run the norm kernel and the tiles:
 their logits agree, at a width below a workgroup's first sweep of the row (256
-threads of 8 columns), at one that ends inside the second and at the widest.
+threads of 8 columns), at one that ends inside the second and at the widest;
+and with one, two (both loaded ahead) and more split-K slabs of O and down to
+add to the residual stream.
 """
 import numpy as np
 import pytest
 
 from mesh_amd import BackendMicrobatchExecutor, DecodeMicrobatchRequest, KVCacheSnapshot
+from tests.test_gpu_gemm_tiles import STORE, SWIGLU, gemm_plan
 from tests.test_gpu_model import make
 from tests.testmodels import geometry, random_weights
 
-pytestmark = pytest.mark.gpu
 
-
+@pytest.mark.gpu
 @pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("rows", [1, 2])
 @pytest.mark.parametrize("heads,kv_heads,head_dim", [(17, 17, 64), (24, 8, 128), (32, 8, 128)])
 def test_few_rows_equal_the_same_rows_of_a_larger_step(heads, kv_heads, head_dim, rows, split):
-    cfg = dict(hidden=heads * head_dim, num_heads=heads, num_kv_heads=kv_heads, num_layers=2, vocab=512, ffn=256,
+    compare_steps(heads, kv_heads, head_dim, 256, rows, split)
+
+
+# (heads, kv heads, head dim, FFN, slabs of O, slabs of down)
+SLABS = [(32, 4, 64, 5632, 2, 2), (16, 16, 64, 4096, 1, 4), (8, 2, 64, 8192, 1, 8)]
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("heads,kv_heads,head_dim,ffn,o,down", SLABS)
+def test_slab_cases_leave_the_slabs_they_name(heads, kv_heads, head_dim, ffn, o, down, rows):
+    h = heads * head_dim
+    assert gemm_plan(rows, h, h, STORE).splits == o and gemm_plan(rows, h, ffn, STORE).splits == down
+    # ... and both products that normalise are unsplit
+    assert gemm_plan(rows, h + 2 * kv_heads * head_dim, h, STORE).direct and gemm_plan(rows, 2 * ffn, h, SWIGLU).direct
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("heads,kv_heads,head_dim,ffn,o,down", SLABS)
+def test_residual_slabs(heads, kv_heads, head_dim, ffn, o, down, rows, split):
+    compare_steps(heads, kv_heads, head_dim, ffn, rows, split)
+
+
+def compare_steps(heads, kv_heads, head_dim, ffn, rows, split):
+    cfg = dict(hidden=heads * head_dim, num_heads=heads, num_kv_heads=kv_heads, num_layers=2, vocab=512, ffn=ffn,
                rms_norm_eps=1e-5, rope_base=10000.0)
     geo = geometry(cfg)
     ctx, _ = make(cfg, geo, random_weights(cfg, geo, seed=7), "f32", split, max_tokens=16, max_seqs=16, pages=256,
