@@ -180,6 +180,22 @@ __global__ __launch_bounds__(plain_max_waves(NB) * 64) void paged_attention_plai
         for (int b = 0; b < NB; ++b) o[t][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
+    // The next page's loads are issued before this page's arithmetic where
+    // both fit the registers of 8 waves per CU (4 above 128 dims), by the
+    // compiler's report, and the columns of a page with values that are not
+    // finite (below) go block by block of dims where a column's whole row of V,
+    // widened at once, would not.  The 32-column forms of 81-128 dims spilled
+    // 180-440 bytes, in the page loop for bf16, and those above 192 dims 112; now
+    // none does, but 88 bytes with 81-96 bf16 dims (reading ahead still gains
+    // there: 1047 us against 1205) and 68 with 113-128 bf16 ones, 184 with f32
+    // ones, both off the loop's straight path.  Two 1000-row chunks on 3000 rows,
+    // us before / now: 32 heads of 96, bf16 1092 / 1047, f32 1572 / 1106; 40 heads
+    // of 128 on 8, bf16 3925 / 1664; 32 heads of 112, bf16 2810 / 1340.
+    constexpr bool kAhead = NB > 8    ? NB < 16
+                            : CT == 2 ? NB < 6 || (NB == 6 && sizeof(KV) == 2)
+                                      : NB < 8 || sizeof(KV) == 2;
+    constexpr bool kByBlock = NB >= 6 && !(NB == 8 && sizeof(KV) == 4);
+
     // keys below `free_end` are visible to every column of the tile
     const int free_end = kvb + c0 / G + 1;
     auto page_step = [&](const PageK<KV, NB>& k, const PageV<KV, NB>& v, int p) {
@@ -236,18 +252,35 @@ __global__ __launch_bounds__(plain_max_waves(NB) * 64) void paged_attention_plai
 #pragma unroll
                 for (int t = 0; t < CT; ++t) {
                     if (t == 1 && !two) continue;
-                    for (int cs = 0; cs < 16; ++cs) {
-                        const int jm = __shfl(jmax[t], cs, 64);
+                    if constexpr (kByBlock) {
 #pragma unroll
-                        for (int b = 0; b < NB; ++b) {
-                            f32x4 x = o[t][b];
+                        for (int b = 0; b < NB; ++b)
+#pragma clang loop unroll(disable)
+                            for (int cs = 0; cs < 16; ++cs) {
+                                const int jm = __shfl(jmax[t], cs, 64);
+                                f32x4 x = o[t][b];
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                const int key = j0 + 4 * q4 + i;
-                                const float vv = key >= 0 && key <= jm ? v.get(i, b) : 0.0f;
-                                x = __builtin_amdgcn_mfma_f32_16x16x4f32(vv, pr[t][i], x, 0, 0, 0);
+                                for (int i = 0; i < 4; ++i) {
+                                    const int key = j0 + 4 * q4 + i;
+                                    const float vv = key >= 0 && key <= jm ? v.get(i, b) : 0.0f;
+                                    x = __builtin_amdgcn_mfma_f32_16x16x4f32(vv, pr[t][i], x, 0, 0, 0);
+                                }
+                                if (c == cs) o[t][b] = x;
                             }
-                            if (c == cs) o[t][b] = x;
+                    } else {
+                        for (int cs = 0; cs < 16; ++cs) {
+                            const int jm = __shfl(jmax[t], cs, 64);
+#pragma unroll
+                            for (int b = 0; b < NB; ++b) {
+                                f32x4 x = o[t][b];
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    const int key = j0 + 4 * q4 + i;
+                                    const float vv = key >= 0 && key <= jm ? v.get(i, b) : 0.0f;
+                                    x = __builtin_amdgcn_mfma_f32_16x16x4f32(vv, pr[t][i], x, 0, 0, 0);
+                                }
+                                if (c == cs) o[t][b] = x;
+                            }
                         }
                     }
                 }
@@ -265,9 +298,6 @@ __global__ __launch_bounds__(plain_max_waves(NB) * 64) void paged_attention_plai
             }
     };
 
-    // The next page's loads are issued before this page's arithmetic where
-    // both fit the registers.
-    constexpr bool kAhead = 8 * CT * NB + 4 * (int)sizeof(KV) * NB <= (NB > 8 ? 400 : 192);
     if constexpr (kAhead) {
         PageK<KV, NB> k[2];
         PageV<KV, NB> v[2];

@@ -7,17 +7,27 @@ Tolerance: every product and sum is f32, as in the reference; a score of D
 products and a weighted sum of L values carry a few rounding errors of 2^-24 of
 their running magnitude.  1e-5 of a row's largest value is over ten times that
 at D = 256 and 700 keys, and far below the 2^-16 of a bf16 hi + lo product."""
+import ctypes as C
 import math
 
 import numpy as np
 import pytest
 
-from mesh_amd import DeviceBuffer, DeviceContext, KVCacheSnapshot, ModelGeometry
+from mesh_amd import DeviceBuffer, DeviceContext, KVCacheSnapshot, ModelGeometry, _lib
 from tests.gpu_util import stage_mixed
 
-pytestmark = pytest.mark.gpu
-
 RTOL = 1e-5
+
+
+class PlainPlan(C.Structure):
+    """zr::PlainAttnPlan (zr_internal.h)."""
+    _fields_ = [("ct", C.c_int), ("waves", C.c_int)]
+
+
+def plain_plan(heads, kv_heads, D, q_len):
+    fn = C.CDLL(_lib.LIB_PATH)._ZN2zr20plain_attention_planEiiiPKii
+    fn.restype = PlainPlan
+    return fn(D, kv_heads, heads // kv_heads, (C.c_int * len(q_len))(*q_len), len(q_len))
 
 
 def bf16(x):
@@ -82,6 +92,7 @@ def reference(seqs, heads, kv_heads, D):
     return np.stack(rows)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("heads,kv_heads,D", [
     (8, 8, 4), (8, 4, 16), (8, 2, 20), (8, 8, 36), (8, 1, 48), (8, 2, 60), (8, 8, 80), (8, 4, 96), (8, 2, 100),
@@ -97,6 +108,7 @@ def test_every_multiple_of_four_head_dim_and_group(kv_dtype, heads, kv_heads, D)
     assert err.max() <= RTOL, np.unravel_index(err.argmax(), err.shape)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("heads,kv_heads,D", [(16, 16, 2), (16, 4, 6), (48, 16, 18), (16, 2, 62), (16, 16, 66),
                                               (16, 2, 98), (16, 8, 126), (16, 16, 130), (16, 4, 190), (16, 2, 254)])
@@ -111,15 +123,19 @@ def test_even_head_dims_that_are_no_multiple_of_four(kv_dtype, heads, kv_heads, 
     assert err.max() <= RTOL, np.unravel_index(err.argmax(), err.shape)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,D,rows", [(32, 32, 80, 200), (32, 8, 96, 90), (16, 4, 256, 60)])
 def test_wide_and_narrow_column_tiles(heads, kv_heads, D, rows):
-    """Chunks long enough for 32-column tiles (up to 128 dims) beside decode rows."""
+    """Chunks beside decode rows: 32-column tiles, 16-column ones where wider
+    ones would leave CUs idle, and the only form above 128 dims."""
+    assert plain_plan(heads, kv_heads, D, [rows, 1]).ct == (2 if D == 80 else 1)
     out, seqs = run_attention(heads, kv_heads, D, "bf16", [(411, rows, 3), (690, 1, 0)], np.random.default_rng(rows))
     want = reference(seqs, heads, kv_heads, D)
     err = np.abs(out - want).reshape(len(out), heads, D).max(-1) / np.abs(want).reshape(len(out), heads, D).max(-1)
     assert err.max() <= RTOL
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
 def test_rows_a_query_does_not_see_never_reach_it(kv_dtype):
     """Infinite and NaN values in rows outside a query's window: later rows of
@@ -146,6 +162,56 @@ def test_rows_a_query_does_not_see_never_reach_it(kv_dtype):
     with np.errstate(invalid="ignore"):
         want = reference(seqs, heads, kv_heads, D)
     assert np.isfinite(want).sum() < want.size and np.isfinite(want[:11]).all() and np.isfinite(want[30:]).all()
+    np.testing.assert_array_equal(np.isfinite(out), np.isfinite(want))
+    fine = np.isfinite(want)
+    np.testing.assert_allclose(out[fine], want[fine], rtol=0, atol=RTOL * np.abs(want[fine]).max())
+
+
+# 32-column tiles: every count of 16-dim blocks they have, its first and its
+# last head dim; (heads, kv heads, D, chunk rows, waves)
+WIDE = [(32, 32, 4, 200, 8), (32, 32, 16, 200, 8), (32, 32, 20, 200, 8), (32, 32, 32, 200, 8), (32, 32, 36, 200, 8),
+        (32, 32, 48, 200, 8), (32, 32, 52, 200, 8), (48, 16, 64, 200, 8), (32, 32, 68, 200, 8), (32, 32, 80, 212, 8),
+        (32, 32, 84, 200, 8), (32, 32, 96, 200, 8), (32, 32, 100, 200, 8), (32, 32, 112, 220, 8),
+        (32, 32, 116, 200, 4), (40, 8, 128, 220, 4), (64, 16, 40, 257, 4), (48, 16, 96, 400, 4)]
+
+
+@pytest.mark.parametrize("heads,kv_heads,D,rows,waves", WIDE)
+def test_wide_cases_take_the_tiles_they_name(heads, kv_heads, D, rows, waves):
+    p = plain_plan(heads, kv_heads, D, [rows, 1])
+    assert (p.ct, p.waves) == (2, waves)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("heads,kv_heads,D,rows,waves", WIDE)
+def test_tiles_of_32_columns(kv_dtype, heads, kv_heads, D, rows, waves):
+    """A chunk on a window trimmed to start mid-page, its last tile narrower
+    than 16 columns or ending inside its second half, beside a decode row."""
+    out, seqs = run_attention(heads, kv_heads, D, kv_dtype, [(150, rows, 3), (690, 1, 0)], np.random.default_rng(D))
+    want = reference(seqs, heads, kv_heads, D)
+    err = np.abs(out - want).reshape(len(out), heads, D).max(-1) / np.abs(want).reshape(len(out), heads, D).max(-1)
+    assert err.max() <= RTOL, np.unravel_index(err.argmax(), err.shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("heads,kv_heads,D", [(32, 32, 20), (32, 32, 80), (48, 16, 96), (32, 32, 112), (40, 8, 128)])
+def test_unseen_rows_in_tiles_of_32_columns(kv_dtype, heads, kv_heads, D):
+    """As test_rows_a_query_does_not_see_never_reach_it, with both column
+    tiles of a workgroup on the page."""
+    rows = 240
+
+    def edit(Ks, Vs):
+        Vs[0][:7] = np.nan
+        Vs[0][7 + 40 + 11, 5] = np.inf   # the chunk's row 11: columns of the first tiles see it or not
+        Vs[0][7 + 40 + 150, 1] = -np.inf
+        Ks[1][:6] = np.inf
+
+    out, seqs = run_attention(heads, kv_heads, D, kv_dtype, [(40, rows, 7), (20, 1, 6)], np.random.default_rng(D), edit)
+    with np.errstate(invalid="ignore"):
+        want = reference(seqs, heads, kv_heads, D)
+    assert plain_plan(heads, kv_heads, D, [rows, 1]).ct == 2
+    assert np.isfinite(want[:11]).all() and not np.isfinite(want[11:rows]).all()
     np.testing.assert_array_equal(np.isfinite(out), np.isfinite(want))
     fine = np.isfinite(want)
     np.testing.assert_allclose(out[fine], want[fine], rtol=0, atol=RTOL * np.abs(want[fine]).max())
