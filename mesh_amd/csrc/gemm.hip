@@ -1081,9 +1081,11 @@ static void few_rows_launch(const GemmPlan& p, hipStream_t stream, const uint16_
 
 // Every workgroup normalises the rows for itself, from L2 and under the flight
 // of its first weights: one or two rows cost a product 0-0.8 us where the norm
-// launch took 3.6, until the rows read again weigh beside the weights (Llama-3
-// gate/up, 1792 workgroups of 16 KB per row and buffer: step of 4 layers with
-// one row 675 -> 659 us, with two 479 -> 492).
+// launch took 3.6.  Llama-3 steps of 4 layers, us per step replayed on three
+// streams / by itself: one row (gate/up 1792 workgroups of 16 KB per row and
+// buffer) 470 / 597 inside, 485 / 628 with norm launches.  Past 2048 rows x
+// workgroups the rows read again weigh beside the weights and nothing more is
+// gained: two rows with gate/up's norms inside 494 / 614, outside 497 / 615.
 bool norm_in_gemm(int m, int n, int k, int epilogue) {
     if (m < 1 || m > kNormRows || k > kNormCols || k % 32 != 0 || !few_rows(m, n, epilogue) ||
         2 * packed_weight_elems(k, n) > 0x7fffffffull)
