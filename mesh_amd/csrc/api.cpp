@@ -120,7 +120,9 @@ static zr_status resolve_geometry(zr_context* ctx) {
 }
 
 // Split-K workspace of one GEMM shape (same plan as launch_gemm).
-static size_t gemm_ws_floats(int m, int n, int k, int epilogue) { return gemm_plan(m, n, k, epilogue).ws_floats; }
+static size_t gemm_ws_floats(int m, int n, int k, int epilogue) {
+    return std::max(gemm_plan(m, n, k, epilogue, false).ws_floats, gemm_plan(m, n, k, epilogue, true).ws_floats);
+}
 
 static void destroy_streams(zr_context* ctx) {
     for (hipStream_t* st : {&ctx->stream, &ctx->d2h_stream, &ctx->h2d_stream})
@@ -584,7 +586,6 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
     if (rc) return rc;
     const zr_model_desc& d = ctx->desc;
     const int T = st->total_q, S = st->num_seqs, H = d.hidden, F = d.ffn_cols;
-    (void)S;
     const int QKV = ctx->q_cols + 2 * ctx->kv_cols;
     if ((rc = launch_embed(ctx, st, d_tokens ? d_tokens : st->tokens, d_tokens != nullptr))) return rc;
     const int lo = (d.flags & ZR_FLAG_SPLIT_ACTIVATIONS) ? 1 : 0;
@@ -593,6 +594,9 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
     Slabs down(nullptr);
     // one or two rows: the norms inside the products that read them, the
     // residual stream alternating between two buffers
+    // decode steps keep the order of their sums whether the call waits or not:
+    // replayed and pipelined steps agree bit for bit
+    const bool waits_alone = waits && T > S;
     const bool norm_qkv = norm_in_gemm(T, QKV, H, kEpiStore);
     const bool norm_gate_up = norm_in_gemm(T, 2 * F, H, kEpiSwiGLU);
     float *hidden = ctx->hidden, *other = ctx->hidden2;
@@ -611,7 +615,8 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
             if ((rc = launch_rms_norm(ctx, hidden, l > 0 ? down : Slabs(nullptr), hidden, L.attn_norm, nullptr,
                                       ctx->xa, lo, nullptr, T, H)))
                 return rc;
-            if ((rc = launch_gemm(ctx, ctx->xa, L.w_qkv, ctx->qkv, nullptr, T, QKV, H, kEpiStore, &qkv))) return rc;
+            if ((rc = launch_gemm(ctx, ctx->xa, L.w_qkv, ctx->qkv, nullptr, T, QKV, H, kEpiStore, &qkv, waits_alone)))
+                return rc;
         }
         if (st->fuse_rope) {  // RoPE + KV append inside the decode attention launch
             if ((rc = launch_attention_rope(ctx, st, l, qkv, 1, nullptr, ctx->attn_a))) return rc;
@@ -621,7 +626,7 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
         }
         Slabs o(ctx->proj);
         if ((rc = launch_gemm(ctx, ctx->attn_a, L.w_o, ctx->proj, nullptr, T, H, ctx->q_cols, kEpiStore,
-                              h_partials ? nullptr : &o)))
+                              h_partials ? nullptr : &o, waits_alone)))
             return rc;
         if (h_partials)
             ZR_HIP(ctx, hipMemcpyAsync(h_partials + ((size_t)l * 2 + 0) * T * H, ctx->proj, sizeof(float) * T * H,
@@ -640,7 +645,8 @@ static zr_status run_forward(zr_context* ctx, StagedMeta* st, const uint32_t* d_
                 return rc;
         }
         down = Slabs(ctx->proj);
-        if ((rc = launch_gemm(ctx, ctx->ffn_a, L.w_down, ctx->proj, nullptr, T, H, F, kEpiStore, defer))) return rc;
+        if ((rc = launch_gemm(ctx, ctx->ffn_a, L.w_down, ctx->proj, nullptr, T, H, F, kEpiStore, defer, waits_alone)))
+            return rc;
         if (h_partials)
             ZR_HIP(ctx, hipMemcpyAsync(h_partials + ((size_t)l * 2 + 1) * T * H, ctx->proj, sizeof(float) * T * H,
                                        hipMemcpyDeviceToHost, ctx->stream));

@@ -921,7 +921,8 @@ static float cu_time(const TileCost& t, int splits, int rows, int n, int k, int 
 // against 2232 with it, 1400 rows 4722 / 4457; TinyLlama, 8 layers, 800 rows
 // 1470 / 1428), and 0-5 % faster where none do.
 // waits: no limit -- the caller waits for this microbatch, and nothing else of
-// its context runs beside it.
+// its context runs beside it (a 760-row Llama-3 prompt of 3 layers 2257 us with
+// the limit, 2199 without).
 static GemmChoice cheapest(int m, int n, int k, int epilogue, const GemmChoice& most, bool waits) {
     const int rows = (m + 63) / 64 * 64, KT = (k + 31) / 32, cus = device_cus();
     auto same = [](const GemmCfg& a, const GemmCfg& b) {
@@ -1007,7 +1008,7 @@ static GemmChoice choose_tiles(int m, int n, int k, int epilogue, bool waits) {
     // down 479 / 456 against 405 / 432, gate/up at 1000 408 / 394 against 380 /
     // 366; TinyLlama at 1000 gate/up 103 / 82 against 88 / 76, at 300 QKV 12.9 /
     // 11.5 against 12.4 / 8.6 with half the slabs.
-    return cheapest(m, n, k, epilogue, plain, false);
+    return cheapest(m, n, k, epilogue, plain, waits);
 }
 
 GemmPlan gemm_plan(int m, int n, int k, int epilogue, bool waits) {

@@ -439,8 +439,10 @@ struct GemmPlan {
     bool direct = true;
     size_t ws_floats = 0;
 };
-// waits: the caller waits for the microbatch; the tiles of a fused gate / up
-// product (not its bits) then follow its time by itself, otherwise its CU time.
+// waits: the caller waits for the microbatch; tiles and K splits over many rows
+// then follow the product's time by itself, otherwise its CU time too.  Of a
+// fused gate / up product that changes no bit, of the others (past 256 rows)
+// the order of the sums.
 GemmPlan gemm_plan(int m, int n, int k, int epilogue, bool waits = false);
 // C = A @ W (W packed, A bf16 operand).  kEpiStore writes c_f32; kEpiSwiGLU
 // writes silu(gate) * up as the bf16 operand c_bf16 (or f32 c_f32).  With

@@ -10,7 +10,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from mesh_amd import BackendMicrobatchExecutor, DeviceBuffer, _lib
+from mesh_amd import BackendMicrobatchExecutor, DeviceBuffer, KVCacheSnapshot, _lib
 from tests import test_gpu_kernels as kernels
 from tests.gpu_util import stage_mixed
 from tests.test_gpu_model import make
@@ -27,7 +27,7 @@ class GemmPlan(C.Structure):
 
 
 def gemm_plan(m, n, k, epilogue, waits=True):
-    """waits: of a call that waits for its microbatch, as the op entries and zr_forward do."""
+    """waits: of a call that waits for its microbatch, as zr_forward and zr_gemm_swiglu do."""
     fn = C.CDLL(_lib.LIB_PATH)._ZN2zr9gemm_planEiiiib
     fn.restype, fn.argtypes = GemmPlan, [C.c_int] * 4 + [C.c_bool]
     return fn(m, n, k, epilogue, waits)
@@ -120,9 +120,8 @@ STORED = [(300, 128, 64, (64, 256), 1, 1),
 
 @pytest.mark.parametrize("m,k,n,shape,splits,left", STORED)
 def test_stored_cases_take_the_tiles_they_name(m, k, n, shape, splits, left):
-    for waits in (True, False):
-        p = gemm_plan(m, n, k, STORE, waits)
-        assert (tile(p), p.splits, p.col_blocks * p.splits % 8) == (shape, splits, left)
+    p = gemm_plan(m, n, k, STORE, False)  # as zr_gemm's
+    assert (tile(p), p.splits, p.col_blocks * p.splits % 8) == (shape, splits, left)
 
 
 @pytest.mark.gpu
@@ -132,40 +131,80 @@ def test_store_tiles(split, m, k, n, shape, splits, left):
     kernels.test_gemm_matches_fp64(split, m, k, n)
 
 
-# Microbatches beside other streams: gate / up takes no more CU time than 128 x
-# 256 tiles (128 x 512 ones that fill two passes), whatever fills a pass better.
-# (rows, k, f, tile of a waiting call, of an asynchronous one)
-BESIDE = [(200, 2048, 5632, (64, 256), (128, 256)), (256, 4096, 7168, (64, 256), (128, 256)),
-          (600, 4096, 14336, (192, 256), (128, 256)), (640, 4096, 7168, (192, 256), (128, 512)),
-          (1400, 4096, 14336, (128, 256), (128, 512)), (997, 2048, 5632, (256, 256), (256, 256))]
+# Microbatches beside other streams take no more CU time than 128 x 256 tiles
+# (128 x 512 ones that fill two passes) would, whatever fills a pass better.
+# (rows, k, n, epilogue, tile and splits of a waiting call, of an asynchronous one)
+BESIDE = [(200, 2048, 11264, SWIGLU, ((64, 256), 1), ((128, 256), 1)),
+          (256, 4096, 14336, SWIGLU, ((64, 256), 1), ((128, 256), 1)),
+          (600, 4096, 28672, SWIGLU, ((192, 256), 1), ((128, 256), 1)),
+          (640, 4096, 14336, SWIGLU, ((192, 256), 1), ((128, 512), 1)),
+          (1400, 4096, 28672, SWIGLU, ((128, 256), 1), ((128, 512), 1)),
+          (997, 2048, 11264, SWIGLU, ((256, 256), 1), ((256, 256), 1)),
+          (700, 4096, 6144, STORE, ((192, 256), 2), ((128, 256), 1)),
+          (2108, 2048, 2048, STORE, ((192, 256), 2), ((128, 256), 1)),
+          (997, 2048, 2560, STORE, ((128, 256), 3), ((128, 256), 3)),
+          (208, 4096, 3072, STORE, ((128, 256), 10), ((128, 256), 10))]  # up to 256 rows: one plan
 
 
-@pytest.mark.parametrize("m,k,f,alone,beside", BESIDE)
-def test_asynchronous_microbatches_take_tiles_by_their_cu_time(m, k, f, alone, beside):
-    plans = [gemm_plan(m, 2 * f, k, SWIGLU, w) for w in (True, False)]
-    assert [tile(p) for p in plans] == [alone, beside]
-    work = {(128, 256): 0.863, (192, 256): 1.232, (256, 256): 1.564, (64, 256): 0.493, (128, 512): 1.62}
-    blocks = -(-m // 128) * (-(-2 * f // 256))
-    assert plans[1].row_blocks * plans[1].col_blocks * work[beside] <= 1.03 * blocks * work[128, 256]
+@pytest.mark.parametrize("m,k,n,epilogue,alone,beside", BESIDE)
+def test_asynchronous_microbatches_take_tiles_by_their_cu_time(m, k, n, epilogue, alone, beside):
+    plans = [gemm_plan(m, n, k, epilogue, w) for w in (True, False)]
+    assert [(tile(p), p.splits) for p in plans] == [alone, beside]
+    if beside[1] == 1:
+        work = {(128, 256): 0.863, (192, 256): 1.232, (256, 256): 1.564, (64, 256): 0.493, (128, 512): 1.62}
+        blocks = -(-m // 128) * -(-n // 256)
+        assert plans[1].row_blocks * plans[1].col_blocks * work[beside[0]] <= 1.03 * blocks * work[128, 256]
+
+
+def both_ways(cfg, lens, chunks, seed, kv_dtype="bf16"):
+    """Logits of one microbatch through zr_forward and through zr_forward_staged_async."""
+    geo = geometry(cfg)
+    ctx, _ = make(cfg, geo, random_weights(cfg, geo, seed=5), kv_dtype, True, max_tokens=1000, max_seqs=len(chunks),
+                  pages=sum((n + c + 15) // 16 + 1 for n, c in zip(lens, chunks)) * 2, pps=80)
+    rng = np.random.default_rng(seed)
+    toks = [rng.integers(0, cfg["vocab"], c).astype(np.uint32) for c in chunks]
+    groups = ([], [])
+    for n in lens:
+        kv = [rng.standard_normal((cfg["num_layers"], n, geo["kv_cols"]), dtype=np.float32) for _ in range(2)]
+        for g in groups:
+            g.append(ctx.new_backend(2048))
+            if n:
+                g[-1].import_kv_cache(KVCacheSnapshot(n, n, *kv))
+    _, waited = BackendMicrobatchExecutor.forward_mixed(groups[0], [t.tolist() for t in toks])
+    st = stage_mixed(ctx, groups[1], chunks, np.concatenate(toks))
+    S, V = len(chunks), cfg["vocab"]
+    d_ids, d_logits = DeviceBuffer(ctx, 4 * S), DeviceBuffer(ctx, 4 * S * V)
+    ctx.check(ctx.lib.zr_forward_staged_async(ctx.h, st, None, d_ids.ptr, d_logits.ptr))
+    ctx.check(ctx.lib.zr_synchronize(ctx.h))
+    got = d_logits.download(np.float32, (S, V))
+    ctx.lib.zr_staged_destroy(st)
+    ctx.close()
+    return waited, got
+
+
+MODEL = dict(hidden=256, num_heads=4, num_kv_heads=2, num_layers=2, vocab=300, ffn=7168, rms_norm_eps=1e-5,
+             rope_base=10000.0)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [200, 700, 1000])
-def test_waiting_and_asynchronous_calls_agree_bit_for_bit(rows):
-    """The tiles differ, the sums do not: one chunk through zr_forward and
-    through zr_forward_staged_async."""
-    cfg = dict(hidden=256, num_heads=4, num_kv_heads=2, num_layers=2, vocab=300, ffn=7168, rms_norm_eps=1e-5,
-               rope_base=10000.0)
-    assert len({tile(gemm_plan(rows, 2 * cfg["ffn"], cfg["hidden"], SWIGLU, w)) for w in (True, False)}) == 2
-    geo = geometry(cfg)
-    ctx, _ = make(cfg, geo, random_weights(cfg, geo, seed=5), "bf16", True, max_tokens=1000, max_seqs=2, pages=256,
-                  pps=80)
-    toks = np.random.default_rng(rows).integers(0, cfg["vocab"], rows).astype(np.uint32)
-    _, want = BackendMicrobatchExecutor.forward_mixed([ctx.new_backend(2048)], [toks.tolist()])
-    st = stage_mixed(ctx, [ctx.new_backend(2048)], [rows], toks)
-    d_ids, d_logits = DeviceBuffer(ctx, 4), DeviceBuffer(ctx, 4 * cfg["vocab"])
-    ctx.check(ctx.lib.zr_forward_staged_async(ctx.h, st, None, d_ids.ptr, d_logits.ptr))
-    ctx.check(ctx.lib.zr_synchronize(ctx.h))
-    np.testing.assert_array_equal(d_logits.download(np.float32, (1, cfg["vocab"])), want)
-    ctx.lib.zr_staged_destroy(st)
-    ctx.close()
+@pytest.mark.parametrize("sessions", [0, 200, 700])
+def test_waiting_and_asynchronous_calls_agree_bit_for_bit(sessions):
+    """Gate / up takes other tiles, whose sums are the same, and a decode step
+    (any row count) or a chunk of up to 256 rows keeps the rest of its plans."""
+    rows = sessions or 200
+    assert len({tile(gemm_plan(rows, 2 * MODEL["ffn"], MODEL["hidden"], SWIGLU, w)) for w in (True, False)}) == 2
+    chunks = [1] * sessions or [rows]
+    waited, got = both_ways(MODEL, [7] * len(chunks) if sessions else [0], chunks, rows)
+    np.testing.assert_array_equal(got, waited)
+
+
+@pytest.mark.gpu
+def test_longer_chunks_agree_but_for_the_order_of_sums():
+    """Past 256 rows a waiting chunk's other products may split K another way."""
+    cfg = dict(MODEL, hidden=4096, num_heads=32, num_kv_heads=8, num_layers=1, ffn=256)
+    assert [gemm_plan(700, 6144, 4096, STORE, w).splits for w in (True, False)] == [2, 1]
+    waited, got = both_ways(cfg, [0], [700], 700, "f32")  # (bf16 K / V rows near a tie would round apart)
+    # operands carry 2^-16 of their value, which sums in another order may round the other way: four products
+    # and the head
+    assert np.isfinite(got).all()
+    assert np.abs(got - waited).max() <= 5 * 2.0 ** -16 * np.abs(waited).max()
