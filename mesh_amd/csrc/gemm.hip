@@ -168,21 +168,16 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(
 
     // (workgroups reach the 8 XCDs round-robin: XCD x runs the pairs x, x + 8,
     // ...; the tiles of the last, fewer than 8, go round all XCDs)
-    const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int groups = col_blocks * splits, whole = (groups >> 3) * row_blocks;
-    int g, rb;
-    if (j < whole) {
-        g = j / row_blocks;
-        rb = j - g * row_blocks;
-        g = 8 * g + x;
-    } else {
-        const int t = (j - whole) * 8 + x;
-        g = t / row_blocks;
-        rb = t - g * row_blocks;
-        g += groups & ~7;
-        if (g >= groups) return;  // padding block
-    }
-    const int cb = g / splits, split = g - cb * splits;
+    // Branch-free and in one unsigned division: this stands before a block's
+    // first copy.
+    const unsigned x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const unsigned groups = (unsigned)(col_blocks * splits), whole = (groups >> 3) * (unsigned)row_blocks;
+    const bool left = j >= whole;
+    const unsigned t = left ? (j - whole) * 8 + x : j, quot = t / (unsigned)row_blocks;
+    const int rb = (int)(t - quot * (unsigned)row_blocks);
+    const unsigned g = left ? (groups & ~7u) + quot : quot * 8 + x;
+    if (g >= groups) return;  // padding block
+    const int cb = (int)(g / (unsigned)splits), split = (int)g - cb * splits;
 
     // the wave index is uniform: readfirstlane keeps it (and every copy
     // offset derived from it) in scalar registers
