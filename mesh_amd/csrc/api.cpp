@@ -215,6 +215,59 @@ static int pages_per_split(const std::vector<int>& tile_pages, int kv_heads) {
     return pps;
 }
 
+// Key tiles per split of prefill blocks with `ktiles[i]` tiles each, or a size
+// that leaves every block whole.  A launch takes its passes over the resident
+// slots, each as long as its longest piece, so the sizes worth trying are the
+// smallest that fit one and two full passes; the tiles per slot alone round up
+// to workgroups that spill into another pass.  Append + attention of one chunk,
+// 32 q / 8 kv heads of 128, bf16 pool, us: whole or splits of at least 32
+// tiles / tiles per slot, at least 8 / this rule: 32 rows on 2000 61 / 46 / 46,
+// 300 on 500 57 / 54 / 53, 300 on 1200 63 / 71 / 59, 500 on 1200 70 / 82 / 70,
+// 700 on none 59 / 69 / 59, 900 on 500 88 / 88 / 77, 544 on 6000 200 / 200 /
+// 150; f32 pool, 400 on 500 - / 80 / 68.
+// Prices in tiles: a pass starts and drains for about 8 and a merge launch takes
+// about 10 (600 rows on none, 19 tiles: 55.7 us whole, 57.1 in two).  At least 8
+// tiles per split (32 heads of 128, 32 rows on 2000: 50 us with 16), and at most
+// 16 splits, which the merge combines in one round trip (32 rows on 6000: 66 us
+// in 24 splits, 53 in 12).
+// A whole step whose launches overlap other streams' pays for the partials and
+// gets no CU time back: 3 chunks of 46 rows on 1394 and 13 decode rows, 3 layers
+// of a Llama-3 shard, 581 us per step against 576 with splits of 16 or more; by
+// itself it takes 680 against 684 (693 with 32).
+int prefill_tiles_per_split(const int* ktiles, int n, int kv_heads, int slots) {
+    constexpr int kWhole = 1 << 30, kPass = 8, kMerge = 10;
+    if (n <= 0 || (long)n * kv_heads >= slots) return kWhole;
+    const int longest = *std::max_element(ktiles, ktiles + n);
+    auto launched = [&](int tps) {
+        long w = 0;
+        for (int i = 0; i < n; ++i) w += (ktiles[i] + tps - 1) / tps;
+        return w * kv_heads;
+    };
+    auto piece = [&](int tps) {  // a block's splits are even: 17 tiles by 8 are 6, 6, 5
+        int most = 0;
+        for (int i = 0; i < n; ++i) {
+            const int ns = (ktiles[i] + tps - 1) / tps;
+            if (ns > 0) most = std::max(most, (ktiles[i] + ns - 1) / ns);
+        }
+        return most;
+    };
+    int best = kWhole;
+    long price = longest + kPass;
+    for (int passes = 1; passes <= 2; ++passes) {
+        int lo = std::max(8, (longest + 15) / 16), hi = longest;  // hi fits: the blocks whole do
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (launched(mid) <= (long)passes * slots)
+                hi = mid;
+            else
+                lo = mid + 1;
+        }
+        const long p = passes * (long)(piece(lo) + kPass) + kMerge;
+        if (p < price) best = lo, price = p;
+    }
+    return best;
+}
+
 zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta* st, const StageFixed* fixed,
                            bool* fits) {
     if (fits) *fits = true;
@@ -308,7 +361,6 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     }
     std::vector<int> tile_pages;
     std::vector<int4> pblk;  // prefill blocks {seq, r0, nrows, pages}
-    long total_ktiles = 0;
     for (int s = 0; s < S && qpt > 0; ++s) {
         const int ql = mb->q_len[s], kb = mb->kv_before[s], fo = mb->first_offset[s];
         if (prows && ql >= prows && (!f32_kv || (long)ql * G * (kb + ql / 2) >= kPrefillF32Work)) {
@@ -317,7 +369,6 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
                 const int last_visible = kb + r0 + nr - 1;
                 const int pages = (fo + last_visible + 1 + kPageRows - 1) / kPageRows;
                 pblk.push_back(make_int4(s, r0, nr, pages));
-                total_ktiles += (pages + 1) / 2;
             }
             continue;
         }
@@ -349,7 +400,7 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     if (const char* env = getenv("ZR_ATTN_PREFILL_KEY_HALVES")) kh = atoi(env) == 1 ? 1 : 2;
     st->prefill_kh = kh;
     // Prefill blocks split along their key tiles (32 keys each) when the
-    // blocks alone leave CUs idle: about 512 / kh workgroups (the resident
+    // blocks alone leave CUs idle: fewer than 512 / kh workgroups (the resident
     // slots: 2 / kh per CU).  Blocks that fill the slots by themselves run
     // unsplit (the 2108-row mixed microbatch, 64 blocks x 8 kv heads, with 4-wave workgroups: 7.82-7.88 ms
     // per microbatch against 7.97-8.02 with 33-tile splits, whose merge takes
@@ -359,19 +410,10 @@ zr_status stage_microbatch(zr_context* ctx, const zr_microbatch* mb, StagedMeta*
     // partials per 16-column group (16 / G rows x G heads, the decode tiles'
     // layout), one item per (group, split) after the decode items, and its
     // groups join the merge list as tiles.
-    // At least 8 tiles per split and at most 16 splits, which the merge
-    // combines in one round trip (append + attention of one chunk, us, with
-    // splits of at least 32 / 16 / 8 tiles; bf16 pool, 32 q / 8 kv heads of 128:
-    // 32 rows on 2000 61 / 50 / 46, on 6000 62 / 53 / 66 (24 splits), 64 on 1500
-    // 58 / 51 / 48, 300 on 500 57 / 56 / 53; f32 pool: 64 on 1500 75 / 62 / 53).
     const long slots = 512 / kh;
-    int tps = (int)std::max<long>(8, (total_ktiles * ctx->local_kv_heads + slots - 1) / slots);
-    int longest = 0;
-    for (const int4& b : pblk) longest = std::max(longest, (b.w + 1) / 2);
-    tps = std::max(tps, (longest + 15) / 16);
-    // (blocks of at most 16 tiles gain less than the merge: 512 rows, 4 kv
-    // heads of 64: 41.8 us whole, 42.6 in two splits)
-    if ((long)pblk.size() * ctx->local_kv_heads >= slots || longest <= 16) tps = 1 << 30;
+    std::vector<int> ktiles;
+    for (const int4& b : pblk) ktiles.push_back((b.w + 1) / 2);
+    int tps = prefill_tiles_per_split(ktiles.data(), (int)ktiles.size(), ctx->local_kv_heads, (int)slots);
     if (const char* env = getenv("ZR_ATTN_PREFILL_TILES_PER_SPLIT")) tps = std::max(1, atoi(env));
     if (G > 16) tps = 1 << 30;  // a 16-column group must hold whole rows
     int next_item = st->n_attn_items;

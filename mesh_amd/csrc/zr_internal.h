@@ -369,6 +369,9 @@ struct StageFixed {
 // Blob bytes of a fixed layout: host part (copied per step) and the whole.
 void stage_fixed_bytes(const zr_context* ctx, int S, int total_q, const StageFixed& f, size_t* host_bytes,
                        size_t* dev_bytes);
+// Key tiles per split of a prefill launch: blocks of ktiles[i] key tiles each,
+// `slots` resident workgroups.
+int prefill_tiles_per_split(const int* ktiles, int n, int kv_heads, int slots);
 // Stages a microbatch.  With `fixed`, a microbatch that is not a pure decode
 // step or exceeds the bucket's capacities sets *fits = false and returns
 // ZR_E_UNSUPPORTED (the caller captures a new bucket).
